@@ -368,17 +368,19 @@ __global__ void __launch_bounds__(kThreads, 2) gg_kernel(Params p) {
     // has landed in every wave and is visible. Each step sums its own stage; the sums meet the end after one more
     // barrier. (A barrier a step, with the DMA three steps ahead, measured 2-3 % slower.)
     // How the wait count is derived (vmcnt counts a wave's vector memory operations and they complete in issue order):
-    //   after its DMA pair (kDmaPerWave each, first in the even step) a wave issues, up to the next even step, the
-    //   codes of two steps (2 after each half's MFMAs, in `compute`: 8) and at most one scale window pair (steps j
-    //   with j % 4 == 3 issue one: 2), kBetween = 10 loads. With at most kBetween outstanding at the top of step k,
-    //   the pair issued at the top of step k - 2 has landed; what may still be out are register loads, which the
-    //   compiler waits for before their first use. A wave with no DMA (!dma_on) has no pair to wait for; the same
+    //   after its DMA pair (kDmaPerWave each, first in the even step) a wave issues, up to the next even step, at
+    //   least the codes of two steps (2 after each half's MFMAs, in `compute`: 8); steps j with j % 4 == 3 issue a
+    //   scale window pair too. The count that is safe is the fewest, kBetween = 8: with at most that many outstanding
+    //   at the top of step k, the pair issued at the top of step k - 2 has landed (with 10, the two more of the steps
+    //   that issue a window, the last two DMA instructions - four rows each - of the steps that issue none could
+    //   still be in flight: four slots of a tile wrong now and then on a cold run). What may still be out are
+    //   register loads, which the compiler waits for before their first use. A wave with no DMA (!dma_on) has no pair to wait for; the same
     //   count only waits for older register loads. The DMA of other waves is covered by their own wait before the
     //   same barrier.
     // A change to what a step issues, or to the order, changes these counts: re-derive them, and run the
     // grouped kernels twice on the same inputs (the parity tests do) - a load landing after its use shows up as
     // run-to-run differences.
-    constexpr int kBetween = 10;
+    constexpr int kBetween = 8;
     auto step = [&](int k, auto st_tag, auto rs_tag, auto two_tag) __attribute__((always_inline)) {
         constexpr int ST = decltype(st_tag)::value;
         if constexpr (ST % 2 == 0) {
@@ -1196,10 +1198,11 @@ __global__ void __launch_bounds__(kGwThreads, 1) gw_kernel(Params p) {
     };
     // One barrier every two K steps: at the top of an even step k every wave has finished steps k - 2 and k - 1
     // (their stages are free) and the DMA of steps k and k + 1 (issued at the top of step k - 2) is visible; the DMA of
-    // steps k + 2 and k + 3 goes out into the freed stages. Wait count: after a DMA pair a wave issues the code loads
-    // of two steps (2 each) and at most one scale window (every fourth step) before the next barrier, so with at most
-    // kBetween loads outstanding the pair has landed (vmcnt counts a wave's loads, completed in issue order).
-    constexpr int kBetween = 5;
+    // steps k + 2 and k + 3 goes out into the freed stages. Wait count: after a DMA pair a wave issues at least the
+    // code loads of two steps (2 each; every other pair of steps a scale window too) before the next barrier, so with
+    // at most those kBetween loads outstanding the pair has landed (vmcnt counts a wave's loads, completed in issue
+    // order).
+    constexpr int kBetween = 4;
     auto step = [&](int k, auto st_tag, auto rs_tag) __attribute__((always_inline)) {
         constexpr int ST = decltype(st_tag)::value;
         if constexpr (ST % 2 == 0) {

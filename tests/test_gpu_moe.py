@@ -344,3 +344,27 @@ def test_combine_grouped_row_counts(d):
     ok = [m for m in range(M) if m != 5]
     ref_y, _ = orc.experts_combine(h[ok], wdn, E, ids[ok], coef[ok])
     util.assert_close(yh[ok], ref_y, what=f"combine_grouped d={d}")
+
+
+# ---------------- grouped experts on a cold run ----------------
+
+@pytest.mark.parametrize("M", [800, 1000])
+def test_grouped_layer_first_run_matches_repeats(M):
+    """The grouped layer's first run (weights and activations cold) gives the same bits as repeated ones: a K step that
+    reads activations still on their way to LDS shows up in the first run only."""
+    import torch
+    from strixite_amd import synthetic as syn
+    from strixite_amd.verify import MoeVerifyLayer
+    E, d, I, k = 512, 4096, 1024, 10
+    layer = MoeVerifyLayer(syn.router_weight(E, d, seed=81), syn.qweight(4, E * 2 * I, d, 128, seed=82),
+                           syn.qweight(4, E * d, I, 128, seed=83), E, k, M)
+    x = syn.activations(M, d, seed=84)
+    sync()
+    print(f"grouped layer, first run against repeats, M={M}", flush=True)
+    first = layer.forward(x).clone()
+    h = layer.h.clone()
+    for _ in range(3):
+        y = layer.forward(x)
+        sync()
+        assert torch.equal(layer.h.view(torch.int16), h.view(torch.int16)), "h of the first run differs"
+        assert torch.equal(y.view(torch.int16), first.view(torch.int16)), "y of the first run differs"
