@@ -5,6 +5,7 @@
 #include "gemm_grouped.hpp"
 #include "dense_ks.hpp"
 #include "qmm.hpp"
+#include "reg_tiles.hpp"
 
 namespace sx {
 namespace {
@@ -129,6 +130,18 @@ int grouped_common(const char *fn, const void *x, const sx_qview *w, int64_t E, 
     return SX_OK;
 }
 
+// Which kernel takes a grouped call: the 64-slot tiles from kPrefillMinTokens tokens and more than kMaxSlotsAnExpert
+// slots an expert on average, the register tiles otherwise (and where the 64-slot ones do not take the shape), qmm for
+// the rest (other group sizes, FP32 activations, long K).
+enum Grouped { kRegTiles, kWideTiles, kQmm };
+Grouped grouped_kernel(const sx_qview *w, int64_t M, int64_t A, int64_t E, int act) {
+    const bool wide = M >= gg::kPrefillMinTokens && gg::eligible(4, w->G, w->K, act) && aligned(w->scale, 4) &&
+                      aligned(w->minv, 4);
+    const bool reg = rt::eligible_grouped(4, w->G, w->N / E, w->K, M, A, E, act);
+    if (reg && !(wide && M * A > rt::kMaxSlotsAnExpert * E)) return kRegTiles;
+    return wide ? kWideTiles : kQmm;
+}
+
 }  // namespace
 }  // namespace sx
 
@@ -221,8 +234,11 @@ int sx_linear_q4_experts_gather_grouped(const void *x, const sx_qview *w, int64_
     if (int rc = grouped_common(fn, x, w, E, M, A, ws, ws_bytes, y, act, math)) return rc;
     const int64_t N = w->N / E, es = act_bytes(act), S = M * A;
     SX_CHECK(apart(x, M * w->K * es, y, S * N * es), fn, " y overlaps x");
-    if (M >= gg::kPrefillMinTokens && gg::eligible(4, w->G, w->K, act) && aligned(w->scale, 4) && aligned(w->minv, 4)) {
-        SX_HIP(gg::launch(qmm::GATHER, x, w, y, static_cast<const int32_t *>(ws), M, A, E, act, stream_of(stream)), fn);
+    const Grouped kernel = grouped_kernel(w, M, A, E, act);
+    const int32_t *route = static_cast<const int32_t *>(ws);
+    if (kernel != kQmm) {
+        SX_HIP(kernel == kRegTiles ? rt::launch_grouped(qmm::GATHER, x, w, y, route, M, A, E, stream_of(stream))
+                                   : gg::launch(qmm::GATHER, x, w, y, route, M, A, E, act, stream_of(stream)), fn);
         return SX_OK;
     }
     Params p{};
@@ -241,8 +257,11 @@ int sx_linear_q4_experts_gather_swiglu_grouped(const void *x, const sx_qview *w,
     const int64_t N = w->N / E, es = act_bytes(act), S = M * A;
     SX_CHECK(N % 2 == 0, fn, " SwiGLU gather needs an even row count per expert ([gate | up]), got ", N);
     SX_CHECK(apart(x, M * w->K * es, h, S * (N / 2) * es), fn, " h overlaps x");
-    if (M >= gg::kPrefillMinTokens && gg::eligible(4, w->G, w->K, act) && aligned(w->scale, 4) && aligned(w->minv, 4)) {
-        SX_HIP(gg::launch(qmm::SWIGLU, x, w, h, static_cast<const int32_t *>(ws), M, A, E, act, stream_of(stream)), fn);
+    const Grouped kernel = grouped_kernel(w, M, A, E, act);
+    const int32_t *route = static_cast<const int32_t *>(ws);
+    if (kernel != kQmm) {
+        SX_HIP(kernel == kRegTiles ? rt::launch_grouped(qmm::SWIGLU, x, w, h, route, M, A, E, stream_of(stream))
+                                   : gg::launch(qmm::SWIGLU, x, w, h, route, M, A, E, act, stream_of(stream)), fn);
         return SX_OK;
     }
     Params p{};
@@ -264,9 +283,11 @@ int sx_linear_q4_experts_combine_grouped(const void *h, const sx_qview *w, int64
     SX_CHECK(apart(y, M * N * es, h, S * w->K * es), fn, " y overlaps h");
     SX_CHECK(apart(y, M * N * es, partial, S * N * 4), fn, " y overlaps partial");
     SX_CHECK(apart(partial, S * N * 4, h, S * w->K * es), fn, " partial overlaps h");
-    if (M >= gg::kPrefillMinTokens && gg::eligible(4, w->G, w->K, act) && aligned(w->scale, 4) && aligned(w->minv, 4)) {
-        SX_HIP(gg::launch(qmm::COMBINE, h, w, partial, static_cast<const int32_t *>(ws), M, A, E, SX_ACT_F32,
-                          stream_of(stream)), fn);
+    const Grouped kernel = grouped_kernel(w, M, A, E, act);
+    const int32_t *route = static_cast<const int32_t *>(ws);
+    if (kernel != kQmm) {
+        SX_HIP(kernel == kRegTiles ? rt::launch_grouped(qmm::COMBINE, h, w, partial, route, M, A, E, stream_of(stream))
+                                   : gg::launch(qmm::COMBINE, h, w, partial, route, M, A, E, SX_ACT_F32, stream_of(stream)), fn);
         return combine_reduce(partial, ids, coef, M, A, E, N, y, act, stream_of(stream));
     }
     Params p{};

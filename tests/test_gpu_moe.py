@@ -368,3 +368,53 @@ def test_grouped_layer_first_run_matches_repeats(M):
         sync()
         assert torch.equal(layer.h.view(torch.int16), h.view(torch.int16)), "h of the first run differs"
         assert torch.equal(y.view(torch.int16), first.view(torch.int16)), "y of the first run differs"
+
+
+# ---------------- grouped experts on the register tiles ----------------
+
+@pytest.mark.parametrize("M,A,E,I,d", [
+    (9, 3, 7, 24, 256),      # two spans a row; a feature tile of 8 of 16
+    (20, 2, 5, 384, 384),    # three spans; buckets around 8 slots
+    (33, 3, 9, 640, 640),    # five spans (one wave a row), 2.5 lines a row; over 32 tokens
+    (17, 2, 4, 768, 768),    # six spans in two slices of four (two spans read twice)
+    (40, 4, 12, 256, 2560),  # five slices; more rounds than blocks: several tiles a block, buckets past 16 slots
+    (24, 3, 6, 272, 2432),   # 19 spans: the last slice overlaps the one before; 17 feature tiles
+    (12, 2, 3, 1536, 1536),  # three slices (six waves)
+    (8, 8, 64, 128, 3584),   # seven slices, one slot a bucket
+    (30, 6, 16, 512, 4096),  # eight slices
+])
+def test_register_tiles_match_oracle(M, A, E, I, d):
+    """Grouped gather, SwiGLU gather and combine at few slots an expert (at most 14 on average): every split of K,
+    partial feature tiles, buckets of 1, 16, 17 and more slots, an invalid id, and the fused SwiGLU bit for bit the
+    separate one."""
+    import torch
+    G = 128
+    rng = np.random.default_rng(M * 1000 + E + d)
+    wgu = util.rand_qweight(rng, 4, E * 2 * I, d, G)
+    x = util.f32_to_bf16(rng.standard_normal((M, d)).astype(np.float32))
+    ids = np.stack([rng.choice(E, A, replace=False) for _ in range(M)]).astype(np.int32)
+    ids[:min(M, 17), 0] = 1                # a bucket of at least 17 slots where M allows
+    ids[M // 2, A - 1] = -1
+    ids_d = torch.from_numpy(ids).cuda()
+    Wgu = kx().QWeight.upload(wgu)
+    xd = util.bf16_dev(x)
+    print(f"register tiles M={M} A={A} E={E} I={I} d={d}", flush=True)
+    ws, err = kx().group_routes(ids_d, E)
+    gu = kx().gather_grouped(xd, Wgu, E, ws, M, A)
+    h = kx().gather_grouped(xd, Wgu, E, ws, M, A, swiglu=True)
+    h2 = kx().swiglu(gu.view(M * A, 2 * I)).view(M, A, I)
+    sync()
+    ref_gu, _ = orc.experts_gather(x, wgu, E, ids)
+    ref_h, _ = orc.experts_gather(x, wgu, E, ids, swiglu=True)
+    util.assert_close(util.host_bits(gu), ref_gu, what="gather")
+    util.assert_close(util.host_bits(h), ref_h, roundings=4, what="gather_swiglu")
+    assert np.array_equal(util.host_bits(h), util.host_bits(h2))
+    assert list(err.cpu().numpy()[:3]) == [1, -1, (M // 2) * A + A - 1]
+    if I % G:
+        return
+    wdn = util.rand_qweight(rng, 4, E * 40, I, G)  # 40 output rows an expert: a partial pair of tiles
+    coef = rng.random((M, A)).astype(np.float32)
+    y = kx().combine_grouped(h, kx().QWeight.upload(wdn), E, ids_d, util.f32_dev(coef), ws)
+    sync()
+    ref_y, _ = orc.experts_combine(util.host_bits(h), wdn, E, ids, coef)
+    util.assert_close(util.host_bits(y), ref_y, what="combine")
