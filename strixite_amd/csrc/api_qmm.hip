@@ -7,6 +7,8 @@
 #include "qmm.hpp"
 #include "reg_tiles.hpp"
 
+#include <cmath>
+
 namespace sx {
 namespace {
 
@@ -71,6 +73,45 @@ int launch_qmm(const char *fn, int mode, int bits, int act_x, int act_y, Params 
     return SX_OK;
 }
 
+enum Kernel { kKSplit, kRegTiles, kWideTiles, kQmm };
+
+// Which kernel takes a dense linear. Up to 16 rows with a power of two of spans: dense_ks. Otherwise the register tiles
+// where they take the shape (reg_tiles.hpp), against
+//   - the 64-token tiles (from dense_min_tokens tokens): above kDenseSplitMaxTokens tokens those; up to there by the two
+//     kernels' times, each linear in its rounds: gs_kernel's 64 x 64 blocks in whole waves of the chip (4096 x 4096, q4
+//     21 us a wave, q8 27), the register tiles' (16 tokens x 32 rows) units a compute unit (q4 7 us and 2.3 each at K =
+//     4096, q8 9 and 4.6), with a fifth in gs_kernel's favour. Both sides measured, register tiles / gs_kernel: q4 4096
+//     x 4096 M = 128 16.2 / 20.4 us, M = 200 26.5 / 21.2; 12288 x 4096 M = 400 98.9 / 120.1; 8192 x 2560 M = 128 18.8 /
+//     15.2; q8 4096 x 4096 M = 48 16.9 / 26.0, 12288 x 4096 M = 64 34.2 / 28.0;
+//   - qmm at short K, where a tile's activations outweigh its weights, and few products (qmm / register tiles: q4 2560 x
+//     640 M = 64 7.9 / 10.7 us, M = 200 12.0 / 11.0; 4096 x 1024 M = 48 7.4 / 9.2, M = 128 10.4 / 9.5; q8 5120 x 2048 M =
+//     18 9.3 / 11.5, where K = 2560 is not on qmm's straight-line path: 7680 x 2560 M = 24 29.3 / 13.9; FP32 rows, 4096 x
+//     1024 M = 128 21.3 / 23.5, M = 300 41.4 / 31.3, q8 1296 x 2048 M = 68 18.7 / 26.2).
+Kernel dense_kernel(int bits, const sx_qview *w, int64_t M, int act, int out_act) {
+    const int64_t N = w->N, K = w->K;
+    const int cus = device_cus();
+    if (dks::eligible(bits, w->G, N, K, M, act, out_act, cus)) return kKSplit;
+    const bool wide = M >= gg::dense_min_tokens(bits) && gg::eligible_dense(bits, w->G, K, act) && aligned(w->scale, 4) &&
+                      aligned(w->minv, 4);
+    if (!rt::eligible_dense(bits, w->G, N, K, M, act)) return wide ? kWideTiles : kQmm;
+    if (wide) {
+        if (M > gg::kDenseSplitMaxTokens) return kWideTiles;
+        const double units = (double)((M + 15) / 16) * (double)((N + 31) / 32) / cus, k = K / 4096.0;
+        const int64_t blocks = (M + 63) / 64 * ((N + 63) / 64);
+        const double waves = (double)((blocks + cus - 1) / cus);
+        const double reg = bits == 4 ? 7 + 2.3 * k * units : 9 + 4.6 * k * ceil(units);
+        const double split = waves * (bits == 4 ? 6 + 15 * k : 4 + 23 * k);
+        return reg * 1.2 < split ? kRegTiles : kWideTiles;
+    }
+    const double macs = (double)M * (double)N * (double)K;
+    bool few;
+    if (act == SX_ACT_F32)
+        few = (bits == 4 ? K <= 1024 : K == 1024) ? macs < 6e8 : bits == 8 && K == 2048 && macs < 4e8;
+    else
+        few = bits == 4 ? K <= 1024 && macs < 3.5e8 : (K == 1024 || K == 2048) && macs < 6e8;
+    return few ? kQmm : kRegTiles;
+}
+
 int linear(const char *fn, int bits, const void *x, const sx_qview *w, void *y, int64_t M, int act, int out_act,
            sx_stream stream) {
     SX_CHECK(x != nullptr && y != nullptr, fn, " null pointer (x=", x, ", y=", y, ")");
@@ -82,16 +123,20 @@ int linear(const char *fn, int bits, const void *x, const sx_qview *w, void *y, 
              " with input ", act, " unsupported (same dtype, or BF16 -> F32)");
     SX_CHECK(apart(x, M * w->K * act_bytes(act), y, M * w->N * act_bytes(out_act)), fn, " output y [", y, ", +",
              M * w->N * act_bytes(out_act), " B) overlaps input x [", x, ", +", M * w->K * act_bytes(act), " B)");
-    if (dks::eligible(bits, w->G, w->N, w->K, M, act, out_act, device_cus())) {  // decode width: K split over a block
+    switch (dense_kernel(bits, w, M, act, out_act)) {
+    case kKSplit: {  // decode width: K split over a block
         dks::Params d{};
         d.x = x, d.q = w->q, d.scale = w->scale, d.minv = w->minv, d.y = y, d.M = (int)M, d.N = w->N, d.K = w->K;
         SX_HIP(dks::launch(bits, w->G, act, out_act, d, device_cus(), stream_of(stream)), fn);
         return SX_OK;
     }
-    if (M >= gg::dense_min_tokens(bits) && gg::eligible_dense(bits, w->G, w->K, act) && aligned(w->scale, 4) &&
-        aligned(w->minv, 4)) {  // prefill width: the grouped kernel's MFMA tiles, the tokens as one bucket
+    case kRegTiles:
+        SX_HIP(rt::launch_dense(bits, x, w, y, M, act, out_act, stream_of(stream)), fn);
+        return SX_OK;
+    case kWideTiles:  // prefill width: the grouped kernel's MFMA tiles, the tokens as one bucket
         SX_HIP(gg::launch_dense(x, w, y, M, out_act, stream_of(stream)), fn);
         return SX_OK;
+    case kQmm: break;
     }
     const int nsplit = act == SX_ACT_F32 ? 3 : 1;
     const int rows = rows_that_fit(bits, nsplit, w->K, w->G, (int)(M < 16 ? M : 16));
@@ -133,8 +178,7 @@ int grouped_common(const char *fn, const void *x, const sx_qview *w, int64_t E, 
 // Which kernel takes a grouped call: the 64-slot tiles from kPrefillMinTokens tokens and more than kMaxSlotsAnExpert
 // slots an expert on average, the register tiles otherwise (and where the 64-slot ones do not take the shape), qmm for
 // the rest (other group sizes, FP32 activations, long K).
-enum Grouped { kRegTiles, kWideTiles, kQmm };
-Grouped grouped_kernel(const sx_qview *w, int64_t M, int64_t A, int64_t E, int act) {
+Kernel grouped_kernel(const sx_qview *w, int64_t M, int64_t A, int64_t E, int act) {
     const bool wide = M >= gg::kPrefillMinTokens && gg::eligible(4, w->G, w->K, act) && aligned(w->scale, 4) &&
                       aligned(w->minv, 4);
     const bool reg = rt::eligible_grouped(4, w->G, w->N / E, w->K, M, A, E, act);
@@ -234,7 +278,7 @@ int sx_linear_q4_experts_gather_grouped(const void *x, const sx_qview *w, int64_
     if (int rc = grouped_common(fn, x, w, E, M, A, ws, ws_bytes, y, act, math)) return rc;
     const int64_t N = w->N / E, es = act_bytes(act), S = M * A;
     SX_CHECK(apart(x, M * w->K * es, y, S * N * es), fn, " y overlaps x");
-    const Grouped kernel = grouped_kernel(w, M, A, E, act);
+    const Kernel kernel = grouped_kernel(w, M, A, E, act);
     const int32_t *route = static_cast<const int32_t *>(ws);
     if (kernel != kQmm) {
         SX_HIP(kernel == kRegTiles ? rt::launch_grouped(qmm::GATHER, x, w, y, route, M, A, E, stream_of(stream))
@@ -257,7 +301,7 @@ int sx_linear_q4_experts_gather_swiglu_grouped(const void *x, const sx_qview *w,
     const int64_t N = w->N / E, es = act_bytes(act), S = M * A;
     SX_CHECK(N % 2 == 0, fn, " SwiGLU gather needs an even row count per expert ([gate | up]), got ", N);
     SX_CHECK(apart(x, M * w->K * es, h, S * (N / 2) * es), fn, " h overlaps x");
-    const Grouped kernel = grouped_kernel(w, M, A, E, act);
+    const Kernel kernel = grouped_kernel(w, M, A, E, act);
     const int32_t *route = static_cast<const int32_t *>(ws);
     if (kernel != kQmm) {
         SX_HIP(kernel == kRegTiles ? rt::launch_grouped(qmm::SWIGLU, x, w, h, route, M, A, E, stream_of(stream))
@@ -283,7 +327,7 @@ int sx_linear_q4_experts_combine_grouped(const void *h, const sx_qview *w, int64
     SX_CHECK(apart(y, M * N * es, h, S * w->K * es), fn, " y overlaps h");
     SX_CHECK(apart(y, M * N * es, partial, S * N * 4), fn, " y overlaps partial");
     SX_CHECK(apart(partial, S * N * 4, h, S * w->K * es), fn, " partial overlaps h");
-    const Grouped kernel = grouped_kernel(w, M, A, E, act);
+    const Kernel kernel = grouped_kernel(w, M, A, E, act);
     const int32_t *route = static_cast<const int32_t *>(ws);
     if (kernel != kQmm) {
         SX_HIP(kernel == kRegTiles ? rt::launch_grouped(qmm::COMBINE, h, w, partial, route, M, A, E, stream_of(stream))

@@ -5,13 +5,13 @@
 namespace sx::gg {
 
 // Tokens from which the grouped entry points take this kernel (the reference switches its grouped path to the WMMA
-// tiles at prefill width; at verify width buckets hold a few slots and qmm's one pass over the weights wins).
+// tiles at prefill width; at verify width buckets hold a few slots and the register tiles' one pass over the weights wins).
 constexpr int64_t kPrefillMinTokens = 32;
 
 bool eligible(int bits, int64_t G, int64_t K, int act);
-// Tokens from which a dense linear takes the MFMA tiles (launch_dense): below, qmm's dense mode is faster. 4096 x
-// 4096, qmm against the K-split tiles (gs_kernel): q4 20.2 / 23.0 us at M = 64, 25.2 / 23.1 at 96; q8 23.7 / 29.3 at
-// 32, 34.0 / 29.5 at 64.
+// Tokens from which launch_dense's tiles can be the faster ones for a dense linear (the rule is in api_qmm.hip): below,
+// their blocks leave most of the chip idle. 4096 x 4096, the register tiles against the K-split tiles (gs_kernel): q4 9.6
+// / 23.0 us at M = 64, 12.8 / 23.1 at 96, 26.5 / 21.2 at 200; q8 16.9 / 26.0 at 48.
 constexpr int64_t kDenseMinTokens = 96, kDenseMinTokensQ8 = 48;
 constexpr int64_t dense_min_tokens(int bits) { return bits == 8 ? kDenseMinTokensQ8 : kDenseMinTokens; }
 // Up to this many tokens launch_dense splits K over each block's waves (gs_kernel): four times the blocks, a quarter

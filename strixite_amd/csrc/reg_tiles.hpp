@@ -17,4 +17,9 @@ bool eligible_grouped(int bits, int64_t G, int64_t N, int64_t K, int64_t M, int6
 hipError_t launch_grouped(int mode, const void *x, const sx_qview *w, void *y, const int32_t *ws, int64_t M, int64_t A,
                           int64_t E, hipStream_t stream);
 
+// A dense linear: q4 G = 128 / q8 G = 64, K of whole spans up to 4096, BF16 or FP32 x (act / out_act as linear's).
+bool eligible_dense(int bits, int64_t G, int64_t N, int64_t K, int64_t M, int act);
+hipError_t launch_dense(int bits, const void *x, const sx_qview *w, void *y, int64_t M, int act, int out_act,
+                        hipStream_t stream);
+
 }  // namespace sx::rt

@@ -78,3 +78,37 @@ def test_linear_k_not_a_whole_span(bits, K, G):
     """K that ends inside the kernels' 64-byte row span (the reference allows any K % G == 0)."""
     got, ref = run(bits, 24, K, G, 3, BF16, F32, seed=K)
     util.assert_close(got, ref, what=f"q{bits} K{K} G{G}")
+
+
+# ---------------- the register tiles ----------------
+
+@pytest.mark.parametrize("bits,act,out_act,M,N,K", [
+    (4, orc.BF16, orc.F32, 1, 40, 2560),      # five slices; a partial pair of row tiles
+    (4, orc.BF16, orc.BF16, 17, 300, 384),    # three spans in one slice; one token in the second tile
+    (4, orc.BF16, orc.F32, 33, 1000, 2432),   # 19 spans: the last slice overlaps the one before
+    (4, orc.BF16, orc.F32, 60, 5000, 2560),   # more units than blocks: whole blocks a tile
+    (4, orc.BF16, orc.BF16, 210, 700, 640),   # many tiles: blocks cross from one tile to the next
+    (4, orc.F32, orc.F32, 5, 33, 4096),       # FP32 rows: exactly one tile of five tokens
+    (4, orc.F32, orc.F32, 11, 520, 3584),     # a last tile of one token; seven slices
+    (8, orc.BF16, orc.F32, 16, 100, 4096),    # eight slices of eight spans
+    (8, orc.BF16, orc.BF16, 6, 4000, 2560),   # five slices, two units a round
+    (8, orc.BF16, orc.F32, 37, 65, 640),      # ten spans in two slices of five
+    (8, orc.BF16, orc.F32, 20, 90, 320),      # five spans in two slices: overlap
+    (8, orc.F32, orc.F32, 37, 300, 2560),
+    (8, orc.F32, orc.F32, 4, 70, 1984),       # 31 spans
+    (8, orc.F32, orc.F32, 130, 700, 1536),
+])
+def test_register_tiles_dense(bits, act, out_act, M, N, K):
+    """linear_q4 / linear_q8 on the register tiles at the edges of their tiles, slices and unit runs, against the oracle;
+    FP32 rows keep their 24 bits (1e-5 of the largest output, as the three-plane kernels)."""
+    import torch
+    from strixite_amd import kernels as kx
+    rng = np.random.default_rng(M + N + K + bits)
+    w = util.rand_qweight(rng, bits, N, K, 128 if bits == 4 else 64)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x = x if act == orc.F32 else util.f32_to_bf16(x)
+    print(f"register tiles q{bits} act={act} out={out_act} M={M} N={N} K={K}", flush=True)
+    y = kx.linear(util.f32_dev(x) if act == orc.F32 else util.bf16_dev(x), kx.QWeight.upload(w), out_act=out_act)
+    torch.cuda.synchronize()
+    util.assert_close(util.host_bits(y), orc.linear_q(x, w, out_act=out_act), tol=1e-5 if out_act == orc.F32 else 1e-3,
+                      what=f"register tiles q{bits} M={M} N={N} K={K}")
