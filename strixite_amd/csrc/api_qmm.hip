@@ -133,7 +133,7 @@ int linear(const char *fn, int bits, const void *x, const sx_qview *w, void *y, 
     case kRegTiles:
         SX_HIP(rt::launch_dense(bits, x, w, y, M, act, out_act, stream_of(stream)), fn);
         return SX_OK;
-    case kWideTiles:  // prefill width: the grouped kernel's MFMA tiles, the tokens as one bucket
+    case kWideTiles:  // prefill width
         SX_HIP(gg::launch_dense(x, w, y, M, out_act, stream_of(stream)), fn);
         return SX_OK;
     case kQmm: break;

@@ -19,6 +19,8 @@
 #include "gemm_grouped.hpp"
 #include "qmm_impl.hpp"
 
+#include <algorithm>
+
 namespace sx::gg {
 namespace {
 
@@ -34,7 +36,7 @@ constexpr int kDmaPerWave = kStageBytes / 1024 / kWaves;  // 16-byte-a-lane DMA 
 constexpr int kMaxGroups = 32;  // K <= 4096: the span sums of every step stay in LDS
 constexpr int kSumStride = kMaxGroups + 4;  // floats a row (16-byte aligned, rows 4 banks apart)
 
-// gg_kernel's K-step layout for q4 (G = 128) and q8 (G = 64) weights: one quantization group a K step (64 bytes of a
+// The kernels' K-step layout for q4 (G = 128) and q8 (G = 64, the dense kernels) weights: one quantization group a K step (64 bytes of a
 // weight row either way), the step's activation rows in 16-byte chunks, chunk c of row r in slot c ^ swz(r). The
 // swizzle makes the 16 rows a quarter-wave's MFMA operand reads touch distinct banks (q4: 256-byte rows, 16 chunks;
 // q8: 128-byte rows, two to the 256 bytes of the banks, so rows r and r + 1 share a swizzle and differ in half).
@@ -62,7 +64,8 @@ struct Params {
     int64_t A, N, K;  // slots a token; rows an expert (SWIGLU: 2I); K
     int64_t E;
     int nrb;  // row blocks
-    int64_t dense_M;  // > 0: a dense linear (GATHER) over dense_M token rows, tile u = tokens 64 u .. (no workspace)
+    int64_t dense_M;  // gs_kernel, gw_kernel: token rows (no workspace)
+    int units, xcd_cus;  // gw_kernel: token tiles x row blocks; compute units an XCD
     int vec_store;    // BF16 output, output rows a multiple of 8 and y 16-byte aligned: stores staged through LDS
 };
 
@@ -123,9 +126,9 @@ __device__ __forceinline__ void dma16(const void *src, void *lds) {
     __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void *)lds, 16, 0, 0);
 }
 
-template <int MODE, typename TY, int BITS>
+template <int MODE, typename TY>
 __global__ void __launch_bounds__(kThreads, 2) gg_kernel(Params p) {
-    using L = Lay<BITS>;
+    using L = Lay<4>;
     constexpr int kSpan = L::kSpan, kStageBytes = L::kStageBytes, kDmaPerWave = L::kDmaPerWave,
                   kSumStride = L::kSumStride;
     // One array a stage, so that the wait-count pass tells a stage's DMA apart from the others'.
@@ -142,13 +145,7 @@ __global__ void __launch_bounds__(kThreads, 2) gg_kernel(Params p) {
     const int E = (int)p.E;
 
     // ---- the 64-slot tile: bucket, slots (wave 0, lane r fills row r) ----
-    if (tid < 64 && p.dense_M > 0) {  // a dense linear: one "bucket" (the weight), the tokens in order
-        const int u = tile_of(blockIdx.x, p.nrb);
-        const int64_t t0 = (int64_t)u * kBM;
-        const int T = t0 < p.dense_M ? (int)min((int64_t)kBM, p.dense_M - t0) : 0;
-        if (lane < T) s_xrow[lane] = (t0 + lane) * K, s_out[lane] = t0 + lane;
-        if (lane == 0) s_T = T, s_bucket = 0;
-    } else if (tid < 64) {
+    if (tid < 64) {
         const int32_t *ws = p.ws;
         const int32_t n_wt = ws[3], S = ws[1];
         int T = 0, bucket = -1;
@@ -188,7 +185,7 @@ __global__ void __launch_bounds__(kThreads, 2) gg_kernel(Params p) {
     __syncthreads();
 
     // ---- this lane's two weight rows (nb = 0, 1), clamped into the expert (stores are masked) ----
-    const int64_t rowbytes = BITS == 4 ? K / 2 : K, ngroups = K / kSpan;
+    const int64_t rowbytes = K / 2, ngroups = K / kSpan;
     const uint8_t *qrow[2];
     const uint16_t *srow[2], *mrow[2];
     int64_t feat[2];
@@ -205,8 +202,8 @@ __global__ void __launch_bounds__(kThreads, 2) gg_kernel(Params p) {
         mrow[nb] = p.minv + row * ngroups;
     }
     // Activation DMA: instruction I covers kDmaRows tile rows from kDmaRows I; lane l writes row kDmaRows I +
-    // l / kChunks, chunk (l % kChunks) ^ swz(row), so slot s of a row holds chunk s ^ swz(row) (q4: 16 instructions
-    // of 4 rows; q8: 8 of 8). This wave issues I = kDmaPerWave wave + i.
+    // l / kChunks, chunk (l % kChunks) ^ swz(row), so slot s of a row holds chunk s ^ swz(row) (16 instructions of
+    // 4 rows). This wave issues I = kDmaPerWave wave + i.
     constexpr int kChunks = L::kChunks, kDmaRows = 64 / kChunks;
     const uint16_t *xl[kDmaPerWave];
 #pragma unroll
@@ -250,23 +247,6 @@ __global__ void __launch_bounds__(kThreads, 2) gg_kernel(Params p) {
     auto sum_rows = [&](int st, int grp) __attribute__((always_inline)) {
         const int r = tid >> 2, qd = tid & 3;
         if (!dma_on) return;  // rows 32..63 of a tile of at most 32 slots
-        if constexpr (BITS == 8) {
-            // chunks 2 qd, 2 qd + 1 in chunk order: slots (2 qd) ^ swz(r) and that ^ 1 (the row is 128-byte aligned)
-            const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char *)(
-                xs_at(st) + r * 128 + (((2 * qd) ^ L::swz(r)) * 16));
-            uint4 raw[2];
-            uint32_t tmp;
-            asm volatile("ds_read_b128 %0, %3\n\t"
-                         "v_xor_b32 %2, 16, %3\n\tds_read_b128 %1, %2\n\ts_waitcnt lgkmcnt(0)"
-                         : "=&v"(raw[0]), "=&v"(raw[1]), "=&v"(tmp)
-                         : "v"(at));
-            float sum = 0.f;
-#pragma unroll
-            for (int i = 0; i < 2; ++i) sum = sum_chunk(raw[i], sum);
-            sum = qmm::detail::group_sum_c<4>(sum);
-            if (qd == 0 && grp < nk) xsum[r * kSumStride + grp] = sum;
-            return;
-        }
         // chunks 4 qd .. 4 qd + 3 of the row in chunk order (chunk c sits in slot c ^ (r & 15)), so that a slot's
         // sum does not depend on its position in the tile
         const uint32_t grp0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char *)(
@@ -324,8 +304,7 @@ __global__ void __launch_bounds__(kThreads, 2) gg_kernel(Params p) {
 #pragma unroll
                 for (int nb = 0; nb < 2; ++nb) {
                     const uint4 &c = cw[RS][nb][half];
-                    if constexpr (BITS == 4) bop[nb] = codes_nat(qmm::detail::dword(c, kq));
-                    else bop[nb] = codes8(qmm::detail::dword(c, 2 * kq), qmm::detail::dword(c, 2 * kq + 1));
+                    bop[nb] = codes_nat(qmm::detail::dword(c, kq));
                 }
 #pragma unroll
                 for (int tb = 0; tb < 2; ++tb) {
@@ -1049,13 +1028,18 @@ __global__ void __launch_bounds__(kThreads, 1) gs_kernel(Params p) {
 // ---------------- dense linear at full prefill width: 128 tokens a wave ----------------
 // gg_kernel's wave owns 64 tokens x 64 rows: each dequantized weight fragment feeds two MFMAs, and the step's VALU
 // work (dequant, the per-span fold, the span sums: ~9 operations an MFMA) is about as long as its MFMAs, which the
-// two waves of a SIMD overlap only in part. Here (dense linears above kDenseSplitMaxTokens tokens: every token tile
-// but the last is full) a block of 8 waves owns 128 tokens x 256 rows, one block a compute unit (two waves a SIMD),
-// and a wave owns 128 tokens x 32 rows as 4 MFMA tiles: each weight fragment feeds four MFMAs, so the dequant an
-// MFMA halves (~5.7 VALU operations an MFMA) for twice the activation operand reads from LDS, and one barrier every
-// two K steps (the block's eight waves meet at each). Otherwise gg_kernel's arithmetic (span sums, fold, the end's span term on the MFMA) for every
-// output: the results are the same bits. Used where its grid fills the chip (128-token tiles x 256-row blocks >= the
-// compute units): 4096 x 4096 at M = 2048, q4 81.8 -> 71.5 us, q8 117.9 -> 91.4 us.
+// two waves of a SIMD overlap only in part. Here (dense linears above kDenseSplitMaxTokens tokens: every token tile but
+// the last is full) a block of 8 waves owns 128 tokens x 256 rows, one block a compute unit (two waves a SIMD), and a wave owns 128 tokens x 32
+// rows as 4 MFMA tiles: each weight fragment feeds four MFMAs, so the dequant an MFMA halves (~5.7 VALU operations an
+// MFMA) for twice the activation operand reads from LDS, and one barrier every two K steps (the block's eight waves meet
+// at each). Otherwise gg_kernel's arithmetic (span sums, fold, the end's span term on the MFMA) for every output: the
+// results are the same bits. 4096 x 4096 at M = 2048, against gg_kernel: q4 81.8 -> 71.5 us, q8 117.9 -> 91.4 us.
+// The units are dealt to the XCDs in equal runs (all of a token tile on one XCD left the fifth to eighth XCD idle for
+// every token tile past a multiple of eight), and an XCD's last round, when at most half full, is split into 64- or
+// 32-token blocks (a step of a 64-token block takes 0.54 of a whole one's time): 7680 x 2560 q4 at M = 1531 93 -> 76 us,
+// 9000 x 3072 M = 1300 159 -> 109, 4096 x 4096 M = 600 51.4 (gg_kernel) -> 41.9, 2560 x 2560 M = 520 33.2 -> 21.5; q8 9000
+// x 2560 M = 1300 172 -> 119. What bounds a whole round: two waves a SIMD of MFMA and VALU work in turn, at a clock that
+// the power limit holds near 2 GHz (8192 x 4096 M = 2048: 0.88 PFLOP/s, 1.02 with x all zero).
 constexpr int kGwThreads = 512, kGwWaves = 8, kGwBM = 128, kGwTB = kGwBM / 32, kGwRows = kGwWaves * 32;
 
 template <int BITS>
@@ -1064,24 +1048,27 @@ struct LayW {
     static constexpr int kDmaPerWave = kStageBytes / 1024 / kGwWaves;  // 4 / 2
 };
 
-template <typename TY, int BITS>
-__global__ void __launch_bounds__(kGwThreads, 1) gw_kernel(Params p) {
+// Of an XCD's n units (128 tokens x 256 rows), its last n % xcd_cus, less than a round of its compute units, are done by
+// two or four blocks a unit (64 or 32 tokens each) where those fit in one round.
+__host__ __device__ inline int gw_split(int n, int xcd_cus) {
+    const int rest = n % xcd_cus;
+    return 4 * rest <= xcd_cus ? 4 : 2 * rest <= xcd_cus ? 2 : 1;
+}
+
+// TB: the block's 32-token tiles (4; 2 or 1 for half or a quarter of a unit).
+template <typename TY, int BITS, int TB>
+__device__ __forceinline__ void gw_run(const Params &p, unsigned char *x0, unsigned char *x1, unsigned char *x2,
+                                       unsigned char *x3, float *xsum, int64_t t0, int64_t r0) {
     using L = Lay<BITS>;
     using W = LayW<BITS>;
-    constexpr int kSpan = L::kSpan, kStageBytes = W::kStageBytes, kDmaPerWave = W::kDmaPerWave,
+    constexpr int kBM = TB * 32, kSpan = L::kSpan, kDmaPerWave = std::max(1, W::kDmaPerWave * TB / kGwTB),
                   kSumStride = L::kSumStride, kChunks = L::kChunks;
-    __shared__ __attribute__((aligned(L::kStageAlign))) unsigned char x0[kStageBytes], x1[kStageBytes],
-        x2[kStageBytes], x3[kStageBytes];
-    __shared__ __attribute__((aligned(16))) float xsum[kGwBM * kSumStride];  // [token][span]
-
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane & 31, h = lane >> 5;
     const int64_t K = p.K, N = p.N, M = p.dense_M;
-    const int64_t t0 = (int64_t)tile_of(blockIdx.x, p.nrb) * kGwBM;
-    if (t0 >= M) return;  // past the tile count: uniform for the block
-    const int T = (int)min((int64_t)kGwBM, M - t0);
-    const int64_t r0 = (int64_t)rowblock_of(blockIdx.x, p.nrb) * kGwRows;
+    if (t0 >= M) return;  // a part past the last tile's tokens: uniform for the block
+    const int T = (int)min((int64_t)kBM, M - t0);
 
     // this lane's weight row, clamped into the weight (stores are masked)
     const int64_t rowbytes = BITS == 4 ? K / 2 : K, ngroups = K / kSpan;
@@ -1102,6 +1089,7 @@ __global__ void __launch_bounds__(kGwThreads, 1) gw_kernel(Params p) {
     const int nk = (int)(K / kSpan);
     auto issue_x = [&](int kstep, int st) __attribute__((always_inline)) {
         const int k = min(kstep, nk - 1);
+        if (kDmaRows * kDmaPerWave * kGwWaves > kBM && kDmaRows * kDmaPerWave * wave >= kBM) return;  // q8, 32 tokens
 #pragma unroll
         for (int i = 0; i < kDmaPerWave; ++i)
             dma16(xl[i] + (int64_t)k * kSpan, xs_at(st) + (kDmaPerWave * wave + i) * 1024);
@@ -1119,6 +1107,7 @@ __global__ void __launch_bounds__(kGwThreads, 1) gw_kernel(Params p) {
     // the reads in asm ending in lgkmcnt(0) (the step's barrier already covers this stage's DMA)
     auto sum_rows = [&](int st, int grp) __attribute__((always_inline)) {
         const int r = tid >> 2, qd = tid & 3;
+        if (TB < kGwTB && r >= kBM) return;  // wave-uniform
         float sum = 0.f;
         if constexpr (BITS == 8) {
             const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char *)(
@@ -1150,18 +1139,18 @@ __global__ void __launch_bounds__(kGwThreads, 1) gw_kernel(Params p) {
         if (qd == 0 && grp < nk) xsum[r * kSumStride + grp] = sum;
     };
 
-    f32x16 acc[kGwTB];
+    f32x16 acc[TB];
 #pragma unroll
-    for (int tb = 0; tb < kGwTB; ++tb) acc[tb] = f32x16{};
+    for (int tb = 0; tb < TB; ++tb) acc[tb] = f32x16{};
     // one K step on stage st with ring slot RS; the ring slot is re-loaded (step k + 2) as its codes are used
     auto compute = [&](int k, int st, auto rs_tag) __attribute__((always_inline)) {
         constexpr int RS = decltype(rs_tag)::value;
         const unsigned char *xb = xs_at(st);
-        f32x16 D[kGwTB];
-        bf16x8 aop[2][kGwTB];  // [buffer][tb], one MFMA step ahead
-        auto load_a = [&](int kk, bf16x8 (&a)[kGwTB]) __attribute__((always_inline)) {
+        f32x16 D[TB];
+        bf16x8 aop[2][TB];  // [buffer][tb], one MFMA step ahead
+        auto load_a = [&](int kk, bf16x8 (&a)[TB]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int tb = 0; tb < kGwTB; ++tb) {
+            for (int tb = 0; tb < TB; ++tb) {
                 const int row = tb * 32 + j;
                 a[tb] = *reinterpret_cast<const bf16x8 *>(xb + row * L::kRowBytes +
                                                           (((h * (kChunks / 2) + kk) ^ L::swz(row)) * 16));
@@ -1179,7 +1168,7 @@ __global__ void __launch_bounds__(kGwThreads, 1) gw_kernel(Params p) {
                 if constexpr (BITS == 4) bop = codes_nat(qmm::detail::dword(c, kq));
                 else bop = codes8(qmm::detail::dword(c, 2 * kq), qmm::detail::dword(c, 2 * kq + 1));
 #pragma unroll
-                for (int tb = 0; tb < kGwTB; ++tb)
+                for (int tb = 0; tb < TB; ++tb)
                     D[tb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aop[kk & 1][tb], bop, kk == 0 ? f32x16{} : D[tb],
                                                                     0, 0, 0);
             }
@@ -1192,7 +1181,7 @@ __global__ void __launch_bounds__(kGwThreads, 1) gw_kernel(Params p) {
             issue_window(k + 5, wnxt);
         }
 #pragma unroll
-        for (int tb = 0; tb < kGwTB; ++tb)
+        for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[tb][v] = fmaf(s_, D[tb][v], acc[tb][v]);
     };
@@ -1269,7 +1258,7 @@ __global__ void __launch_bounds__(kGwThreads, 1) gw_kernel(Params p) {
             split3(cmv, bt);
         }
 #pragma unroll
-        for (int tb = 0; tb < kGwTB; ++tb) {
+        for (int tb = 0; tb < TB; ++tb) {
             float xv[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) xv[e] = gl + e < nk ? xsum[(tb * 32 + j) * kSumStride + gl + e] : 0.f;
@@ -1285,12 +1274,12 @@ __global__ void __launch_bounds__(kGwThreads, 1) gw_kernel(Params p) {
     // stores: tile tb, lane value v = token tb * 32 + 8 (v / 4) + 4 h + v % 4, row j of the wave's 32
     if constexpr (sizeof(TY) == 2) {
         if (p.vec_store) {  // BF16 through LDS (every wave is past its K loop and has drained its DMA: the barrier)
-            constexpr int kRowB = 32 * 2, kChunksRow = 4, kWaveB = kGwBM * kRowB;  // 8 KB a wave
+            constexpr int kRowB = 32 * 2, kChunksRow = 4, kWaveB = kBM * kRowB;  // 8 KB a wave
             static_assert(2 * kWaveB <= kStageBytes, "two waves' staged outputs fit a stage array");
             asm volatile("s_barrier" ::: "memory");
             unsigned char *stg = xs_at(wave >> 1) + (wave & 1) * kWaveB;
 #pragma unroll
-            for (int tb = 0; tb < kGwTB; ++tb)
+            for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
                 for (int v = 0; v < 16; ++v) {
                     const int r = tb * 32 + 8 * (v / 4) + 4 * h + v % 4;
@@ -1299,7 +1288,7 @@ __global__ void __launch_bounds__(kGwThreads, 1) gw_kernel(Params p) {
             const int64_t fbase = r0 + wave * 32;
             TY *hy = static_cast<TY *>(p.y);
 #pragma unroll
-            for (int i = 0; i < kGwBM * kChunksRow / 64; ++i) {
+            for (int i = 0; i < kBM * kChunksRow / 64; ++i) {
                 const int c = lane + 64 * i, r = c / kChunksRow, cc = c % kChunksRow;
                 const int64_t f = fbase + cc * 8;  // N % 8 == 0: a chunk is wholly in or out
                 const uint4 val = *reinterpret_cast<const uint4 *>(stg + r * kRowB + cc * 16);
@@ -1310,7 +1299,7 @@ __global__ void __launch_bounds__(kGwThreads, 1) gw_kernel(Params p) {
     }
     if (feat >= N) return;
 #pragma unroll
-    for (int tb = 0; tb < kGwTB; ++tb)
+    for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             const int r = tb * 32 + 8 * (v / 4) + 4 * h + v % 4;
@@ -1318,9 +1307,34 @@ __global__ void __launch_bounds__(kGwThreads, 1) gw_kernel(Params p) {
         }
 }
 
-template <int MODE, typename TY, int BITS = 4>
+
+template <typename TY, int BITS>
+__global__ void __launch_bounds__(kGwThreads, 1) gw_kernel(Params p) {
+    using L = Lay<BITS>;
+    constexpr int kStageBytes = LayW<BITS>::kStageBytes;
+    __shared__ __attribute__((aligned(L::kStageAlign))) unsigned char x0[kStageBytes], x1[kStageBytes],
+        x2[kStageBytes], x3[kStageBytes];
+    __shared__ __attribute__((aligned(16))) float xsum[kGwBM * L::kSumStride];  // [token][span]
+    // XCD id % 8 takes an equal run of the units (row blocks inside token tiles), whole ones first
+    const int xcd = blockIdx.x % 8, units = p.units;
+    const int u0 = xcd * units / 8, n = (xcd + 1) * units / 8 - u0;
+    const int split = gw_split(n, p.xcd_cus), whole = n - n % p.xcd_cus;
+    int u = blockIdx.x / 8, part = 0;
+    const bool parted = split > 1 && u >= whole;
+    if (parted) part = (u - whole) % split, u = whole + (u - whole) / split;
+    if (u >= n) return;
+    u += u0;
+    const int64_t r0 = (int64_t)(u % p.nrb) * kGwRows;
+    int64_t t0 = (int64_t)(u / p.nrb) * kGwBM;
+    if (!parted) return gw_run<TY, BITS, kGwTB>(p, x0, x1, x2, x3, xsum, t0, r0);
+    t0 += part * (kGwBM / split);
+    if (split == 2) gw_run<TY, BITS, kGwTB / 2>(p, x0, x1, x2, x3, xsum, t0, r0);
+    else gw_run<TY, BITS, kGwTB / 4>(p, x0, x1, x2, x3, xsum, t0, r0);
+}
+
+template <int MODE, typename TY>
 hipError_t go(const Params &p, dim3 grid, hipStream_t stream) {
-    hipLaunchKernelGGL((gg_kernel<MODE, TY, BITS>), grid, dim3(kThreads), 0, stream, p);
+    hipLaunchKernelGGL((gg_kernel<MODE, TY>), grid, dim3(kThreads), 0, stream, p);
     return hipGetLastError();
 }
 
@@ -1332,10 +1346,8 @@ hipError_t launch_dense(const void *x, const sx_qview *w, void *y, int64_t M, in
     p.scale = static_cast<const uint16_t *>(w->scale), p.minv = static_cast<const uint16_t *>(w->minv);
     p.y = y, p.ws = nullptr, p.A = 1, p.N = w->N, p.K = w->K, p.E = 1, p.dense_M = M;
     p.vec_store = out_act == SX_ACT_BF16 && p.N % 8 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
-    p.nrb = (int)((p.N + kWaves * 64 - 1) / (kWaves * 64));
-    const int64_t tiles = (M + kBM - 1) / kBM;
     if (M <= kDenseSplitMaxTokens) {  // K split over each block's waves
-        const dim3 gs_grid((unsigned)(tiles * ((p.N + 63) / 64)));
+        const dim3 gs_grid((unsigned)((M + kBM - 1) / kBM * ((p.N + 63) / 64)));
         auto gs = [&](auto tag, auto bits) {
             hipLaunchKernelGGL((gs_kernel<decltype(tag), decltype(bits)::value>), gs_grid, dim3(kThreads), 0, stream, p);
             return hipGetLastError();
@@ -1346,26 +1358,20 @@ hipError_t launch_dense(const void *x, const sx_qview *w, void *y, int64_t M, in
         return out_act == SX_ACT_F32 ? gs(float{}, std::integral_constant<int, 4>{})
                                      : gs(uint16_t{}, std::integral_constant<int, 4>{});
     }
-    const int64_t wt = (M + kGwBM - 1) / kGwBM, nrb_w = (p.N + kGwRows - 1) / kGwRows;
-    if (wt * nrb_w >= device_cus()) {  // 128 tokens a wave where that grid fills the chip
-        p.nrb = (int)nrb_w;
-        const dim3 gw_grid((unsigned)((wt + 7) / 8 * 8 * nrb_w));
-        auto gw = [&](auto tag, auto bits) {
-            hipLaunchKernelGGL((gw_kernel<decltype(tag), decltype(bits)::value>), gw_grid, dim3(kGwThreads), 0, stream,
-                               p);
-            return hipGetLastError();
-        };
-        if (w->G == 64)
-            return out_act == SX_ACT_F32 ? gw(float{}, std::integral_constant<int, 8>{})
-                                         : gw(uint16_t{}, std::integral_constant<int, 8>{});
-        return out_act == SX_ACT_F32 ? gw(float{}, std::integral_constant<int, 4>{})
-                                     : gw(uint16_t{}, std::integral_constant<int, 4>{});
-    }
-    const dim3 grid((unsigned)((tiles + 7) / 8 * 8 * p.nrb));
-    if (w->G == 64)  // q8
-        return out_act == SX_ACT_F32 ? go<qmm::GATHER, float, 8>(p, grid, stream)
-                                     : go<qmm::GATHER, uint16_t, 8>(p, grid, stream);
-    return out_act == SX_ACT_F32 ? go<qmm::GATHER, float>(p, grid, stream) : go<qmm::GATHER, uint16_t>(p, grid, stream);
+    p.nrb = (int)((p.N + kGwRows - 1) / kGwRows), p.xcd_cus = std::max(1, device_cus() / 8);
+    p.units = (int)((M + kGwBM - 1) / kGwBM * p.nrb);
+    auto blocks = [&](int n) { return n + (gw_split(n, p.xcd_cus) - 1) * (n % p.xcd_cus); };
+    const int n = (p.units + 7) / 8;  // an XCD's units: n or n - 1
+    const dim3 gw_grid((unsigned)(std::max(blocks(n), blocks(n - 1)) * 8));
+    auto gw = [&](auto tag, auto bits) {
+        hipLaunchKernelGGL((gw_kernel<decltype(tag), decltype(bits)::value>), gw_grid, dim3(kGwThreads), 0, stream, p);
+        return hipGetLastError();
+    };
+    if (w->G == 64)
+        return out_act == SX_ACT_F32 ? gw(float{}, std::integral_constant<int, 8>{})
+                                     : gw(uint16_t{}, std::integral_constant<int, 8>{});
+    return out_act == SX_ACT_F32 ? gw(float{}, std::integral_constant<int, 4>{})
+                                 : gw(uint16_t{}, std::integral_constant<int, 4>{});
 }
 
 bool eligible(int bits, int64_t G, int64_t K, int act) {

@@ -10,13 +10,15 @@ constexpr int64_t kPrefillMinTokens = 32;
 
 bool eligible(int bits, int64_t G, int64_t K, int act);
 // Tokens from which launch_dense's tiles can be the faster ones for a dense linear (the rule is in api_qmm.hip): below,
-// their blocks leave most of the chip idle. 4096 x 4096, the register tiles against the K-split tiles (gs_kernel): q4 9.6
-// / 23.0 us at M = 64, 12.8 / 23.1 at 96, 26.5 / 21.2 at 200; q8 16.9 / 26.0 at 48.
+// their blocks leave most of the chip idle. 4096 x 4096, the register tiles against the K-split tiles (gs_kernel): q4
+// 12.4 / 23.0 us at M = 64, 17.2 / 23.1 at 96, 26.5 / 21.2 at 200; q8 16.9 / 26.0 at 48.
 constexpr int64_t kDenseMinTokens = 96, kDenseMinTokensQ8 = 48;
 constexpr int64_t dense_min_tokens(int bits) { return bits == 8 ? kDenseMinTokensQ8 : kDenseMinTokens; }
-// Up to this many tokens launch_dense splits K over each block's waves (gs_kernel): four times the blocks, a quarter
-// of the steps each. 4096 x 4096, gs_kernel against gg_kernel: q4 23.5 / 51.5 us at M = 256, 45.9 / 52.0 at 512,
-// 90.4 / 53.2 at 1024; q8 31.3 / 82.5 at 256, 60.8 / 83.2 at 512, 119.8 / 83.5 at 1024.
+// Up to this many tokens launch_dense splits K over each block's waves (gs_kernel: 64 x 64 tiles, a quarter of the steps
+// each); above, 128-token units (gw_kernel). 4096 x 4096, gs_kernel / gw_kernel: q4 25.0 / 33.6 us at M = 256, 47.4 / 40.1
+// at 512; q8 28.7 / 55.3, 55.3 / 58.6. Where gs_kernel needs three rounds and more (q4
+// 8192 x 2560 M = 512 59.7 / 32.1) gw_kernel would be faster from fewer tokens, but its sums over the whole K round more
+// (FP32 outputs 2.9e-6 against 1.7e-6 of the norm), so those stay.
 constexpr int64_t kDenseSplitMaxTokens = 512;
 // The dense linears the tiles take: eligible's q4, and q8 (G = 64, K % 256 == 0, K <= 4096, BF16 x).
 bool eligible_dense(int bits, int64_t G, int64_t K, int act);

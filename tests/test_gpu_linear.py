@@ -112,3 +112,19 @@ def test_register_tiles_dense(bits, act, out_act, M, N, K):
     torch.cuda.synchronize()
     util.assert_close(util.host_bits(y), orc.linear_q(x, w, out_act=out_act), tol=1e-5 if out_act == orc.F32 else 1e-3,
                       what=f"register tiles q{bits} M={M} N={N} K={K}")
+
+
+# ---------------- the 128-token units: whole rounds and split last rounds ----------------
+
+@pytest.mark.parametrize("bits,out_act,M,N,K", [
+    (4, orc.BF16, 520, 300, 512),     # quarters: a unit or two an XCD; 8 tokens and three empty parts in the last tile
+    (4, orc.F32, 700, 4000, 512),     # halves: 12 units an XCD; 60 tokens and an empty half in the last tile
+    (4, orc.BF16, 1290, 6300, 512),   # a whole round and quarters
+    (4, orc.F32, 1100, 9999, 512),    # a whole round and halves; odd rows: the scattered stores
+    (8, orc.F32, 545, 200, 256),      # q8 quarters: half of the waves stage no activations
+    (8, orc.BF16, 900, 2600, 512),    # q8 halves
+])
+def test_prefill_units(bits, out_act, M, N, K):
+    """Dense linears above the K-split tiles' widths, at every way an XCD's last round of units is split."""
+    y, ref = run(bits, N, K, 128 if bits == 4 else 64, M, orc.BF16, out_act, seed=M + N)
+    util.assert_close(y, ref, tol=1e-5 if out_act == orc.F32 else 1e-3, what=f"prefill units q{bits} M={M} N={N} K={K}")
