@@ -85,8 +85,9 @@ enum Kernel { kKSplit, kRegTiles, kWideTiles, kQmm };
 //     15.2; q8 4096 x 4096 M = 48 16.9 / 26.0, 12288 x 4096 M = 64 34.2 / 28.0;
 //   - qmm at short K, where a tile's activations outweigh its weights, and few products (qmm / register tiles: q4 2560 x
 //     640 M = 64 7.9 / 10.7 us, M = 200 12.0 / 11.0; 4096 x 1024 M = 48 7.4 / 9.2, M = 128 10.4 / 9.5; q8 5120 x 2048 M =
-//     18 9.3 / 11.5, where K = 2560 is not on qmm's straight-line path: 7680 x 2560 M = 24 29.3 / 13.9; FP32 rows, 4096 x
-//     1024 M = 128 21.3 / 23.5, M = 300 41.4 / 31.3, q8 1296 x 2048 M = 68 18.7 / 26.2).
+//     18 9.3 / 11.5, 10752 x 2048 M = 36 14.4 / 17.5, 14000 x 2048 M = 40 26.9 / 21.6, where K = 2560 is not on qmm's
+//     straight-line path: 7680 x 2560 M = 24 29.3 / 13.9; FP32 rows, 4096 x 1024 M = 128 21.3 / 23.5, M = 300 41.4 / 31.3,
+//     q8 1296 x 2048 M = 68 18.7 / 26.2).
 Kernel dense_kernel(int bits, const sx_qview *w, int64_t M, int act, int out_act) {
     const int64_t N = w->N, K = w->K;
     const int cus = device_cus();
@@ -108,7 +109,7 @@ Kernel dense_kernel(int bits, const sx_qview *w, int64_t M, int act, int out_act
     if (act == SX_ACT_F32)
         few = (bits == 4 ? K <= 1024 : K == 1024) ? macs < 6e8 : bits == 8 && K == 2048 && macs < 4e8;
     else
-        few = bits == 4 ? K <= 1024 && macs < 3.5e8 : (K == 1024 || K == 2048) && macs < 6e8;
+        few = bits == 4 ? K <= 1024 && macs < 3.5e8 : (K == 1024 || K == 2048) && macs < 9e8;
     return few ? kQmm : kRegTiles;
 }
 

@@ -1028,18 +1028,19 @@ __global__ void __launch_bounds__(kThreads, 1) gs_kernel(Params p) {
 // ---------------- dense linear at full prefill width: 128 tokens a wave ----------------
 // gg_kernel's wave owns 64 tokens x 64 rows: each dequantized weight fragment feeds two MFMAs, and the step's VALU
 // work (dequant, the per-span fold, the span sums: ~9 operations an MFMA) is about as long as its MFMAs, which the
-// two waves of a SIMD overlap only in part. Here (dense linears above kDenseSplitMaxTokens tokens: every token tile but
-// the last is full) a block of 8 waves owns 128 tokens x 256 rows, one block a compute unit (two waves a SIMD), and a wave owns 128 tokens x 32
-// rows as 4 MFMA tiles: each weight fragment feeds four MFMAs, so the dequant an MFMA halves (~5.7 VALU operations an
-// MFMA) for twice the activation operand reads from LDS, and one barrier every two K steps (the block's eight waves meet
-// at each). Otherwise gg_kernel's arithmetic (span sums, fold, the end's span term on the MFMA) for every output: the
-// results are the same bits. 4096 x 4096 at M = 2048, against gg_kernel: q4 81.8 -> 71.5 us, q8 117.9 -> 91.4 us.
+// two waves of a SIMD overlap only in part. Here (dense linears above kDenseSplitMaxTokens tokens: every token tile
+// but the last is full) a block of 8 waves owns 128 tokens x 256 rows, one block a compute unit (two waves a SIMD),
+// and a wave owns 128 tokens x 32 rows as 4 MFMA tiles: each weight fragment feeds four MFMAs, so the dequant an MFMA
+// halves (~5.7 VALU operations an MFMA) for twice the activation operand reads from LDS, and one barrier every two K
+// steps (the block's eight waves meet at each). Otherwise gg_kernel's arithmetic (span sums, fold, the end's span
+// term on the MFMA) for every output: the results are the same bits. 4096 x 4096 at M = 2048, against gg_kernel: q4
+// 81.8 -> 71.5 us, q8 117.9 -> 91.4 us.
 // The units are dealt to the XCDs in equal runs (all of a token tile on one XCD left the fifth to eighth XCD idle for
 // every token tile past a multiple of eight), and an XCD's last round, when at most half full, is split into 64- or
-// 32-token blocks (a step of a 64-token block takes 0.54 of a whole one's time): 7680 x 2560 q4 at M = 1531 93 -> 76 us,
-// 9000 x 3072 M = 1300 159 -> 109, 4096 x 4096 M = 600 51.4 (gg_kernel) -> 41.9, 2560 x 2560 M = 520 33.2 -> 21.5; q8 9000
-// x 2560 M = 1300 172 -> 119. What bounds a whole round: two waves a SIMD of MFMA and VALU work in turn, at a clock that
-// the power limit holds near 2 GHz (8192 x 4096 M = 2048: 0.88 PFLOP/s, 1.02 with x all zero).
+// 32-token blocks (a step of a 64-token block takes 0.54 of a whole one's time): 7680 x 2560 q4 at M = 1531 93 -> 76
+// us, 9000 x 3072 M = 1300 159 -> 109, 4096 x 4096 M = 600 51.4 (gg_kernel) -> 41.9, 2560 x 2560 M = 520 33.2 ->
+// 21.5; q8 9000 x 2560 M = 1300 172 -> 119. What bounds a whole round: two waves a SIMD of MFMA and VALU work in
+// turn, at a clock that the power limit holds near 2 GHz (8192 x 4096 M = 2048: 0.88 PFLOP/s, 1.02 with x all zero).
 constexpr int kGwThreads = 512, kGwWaves = 8, kGwBM = 128, kGwTB = kGwBM / 32, kGwRows = kGwWaves * 32;
 
 template <int BITS>
