@@ -48,6 +48,10 @@ const char *sx_version(void);
  * kernels/linear_q4.hpp:26-30 and kernels/linear_q8.hpp:13-14. out_act == act, or BF16 x -> F32 y. */
 int sx_linear_q4(const void *x, const sx_qview *w, void *y, int64_t M, int act, int out_act, sx_stream stream);
 int sx_linear_q8(const void *x, const sx_qview *w, void *y, int64_t M, int act, int out_act, sx_stream stream);
+/* The kernel such a call runs on a device of `cus` compute units (<= 0: the current device), without running it: "k_split",
+ * "register_tiles", "wide_tiles_k_split", "wide_tiles" or "qmm"; NULL for a view or width no call takes (sx_last_error).
+ * For tests and profiles; no reference counterpart. */
+const char *sx_linear_kernel(const sx_qview *w, int bits, int64_t M, int act, int out_act, int cus);
 
 /* ---- per-slot MoE experts (decode / short verify), kernels/linear_q4.hpp:32-58 ----
  * w: E experts stacked [E*N, K]; ids [M, A] int32 device. err: >= 3 zeroed uint32 (device).

@@ -7,6 +7,7 @@
 #include "qmm.hpp"
 #include "reg_tiles.hpp"
 
+#include <algorithm>
 #include <cmath>
 
 namespace sx {
@@ -55,8 +56,8 @@ int rows_that_fit(int bits, int nsplit, int64_t K, int64_t G, int want, size_t b
 }
 
 // Tiles a block covers: 4 waves x tiles a wave, enough waves for the chip (~8 a CU) but no more than the work.
-int tiles_per_chunk(int64_t total_tiles) {
-    const int64_t waves = (int64_t)device_cus() * 8;
+int tiles_per_chunk(int64_t total_tiles, int cus) {
+    const int64_t waves = (int64_t)cus * 8;
     int64_t tpw = (total_tiles + waves - 1) / waves;
     tpw = tpw < 1 ? 1 : tpw > 16 ? 16 : tpw;
     return (int)(tpw * qmm::kWaves);
@@ -65,7 +66,7 @@ int tiles_per_chunk(int64_t total_tiles) {
 int launch_qmm(const char *fn, int mode, int bits, int act_x, int act_y, Params &p, int64_t units, int64_t rows_out,
                int64_t grid_y, hipStream_t stream) {
     const int64_t tiles = (rows_out + qmm::kTile - 1) / qmm::kTile;
-    p.tiles_per_chunk = tiles_per_chunk(tiles * units);
+    p.tiles_per_chunk = tiles_per_chunk(tiles * units, device_cus());
     p.nchunks = (int)((tiles + p.tiles_per_chunk - 1) / p.tiles_per_chunk);
     const int64_t gx = units * p.nchunks;
     SX_CHECK(gx >= 1 && gx <= 0x7fffffff && grid_y <= 65535, fn, " grid ", gx, " x ", grid_y, " out of range");
@@ -75,6 +76,49 @@ int launch_qmm(const char *fn, int mode, int bits, int act_x, int act_y, Params 
 
 enum Kernel { kKSplit, kRegTiles, kWideTiles, kQmm };
 
+// Whether qmm takes a dense linear rather than the register tiles, which read a tile's rows of x into each wave's registers
+// first: at short K that costs more than the tile's weights. The lines are in qmm's blocks a compute unit (staged rows x 4
+// waves' weight tiles a block), which its time follows. Both sides measured, qmm / register tiles in us:
+//   - on qmm's straight-line path: up to three blocks a compute unit (two at K = 2048), FP32 rows four and at K = 512 any
+//     number. q8 5120 x 512 M = 24 5.3 / 11.8, 8192 x 1024 M = 37 9.5 / 11.9, 14000 x 2048 M = 24 15.7 / 16.4, M = 32 22.9 /
+//     16.6; q4 8192 x 1024 M = 64 7.8 / 9.6, 14000 x 1024 M = 95 18.4 / 14.8; FP32 rows, q8 5120 x 1024 M = 37 13.8 /
+//     18.9, 8192 x 512 M = 200 26.9 / 38.9, 8192 x 1024 M = 128 47.4 / 42.2. At K = 4096 only as one block a compute unit
+//     where the register tiles need two rounds (5120 x 4096 M = 17 q4 10.1 / 11.6, q8 15.0 / 17.1);
+//   - on its general path below K = 1024, where a block of register tiles holds more than four times the x it needs (each
+//     of its output units has its own, and slices may overlap), for one round of blocks (two where it holds more than 8 KB
+//     a row): q8 5120 x 768 M = 24 10.3 / 11.3, 14000 x 768 M = 24 14.7 / 12.1; q4 5120 x 640 M = 37 8.1 / 10.9, 5120 x 640 M =
+//     200 19.0 / 14.0. FP32 rows, which the register tiles read in more tiles: two rounds, with a bar that rises with the
+//     rows qmm stages, less where the register tiles need a second round: q8 5120 x 768 M = 6 12.9 / 14.3, 5120 x 896 M = 32
+//     15.8 / 19.1, 1000 x 896 M = 24 15.8 / 14.4; slices that overlap by half any number (q8 5120 x 320 M = 200 20.7 / 28.5);
+//   - FP32 rows whose 5-token tiles are more than an eighth of the chip, so that a block passes from tile to tile and
+//     reads x again: q4 2560 x 512 M = 300 17.4 / 23.8, 1000 x 1152 M = 200 16.9 / 22.3; and a single FP32 row up to K = 1280
+//     (q4 8192 x 1152 M = 1 10.4 / 11.1).
+bool qmm_is_faster(int bits, const sx_qview *w, int64_t M, int act, int cus) {
+    const bool f32 = act == SX_ACT_F32;
+    const int64_t K = w->K, span = bits == 4 ? 128 : 64, nspan = K / span;
+    const rt::Block b = rt::dense_block(bits, K, act);
+    const int64_t reg_tiles = (M + (f32 ? 4 : 15)) / (f32 ? 5 : 16);
+    const int64_t reg_rounds = reg_tiles * (((w->N + 31) / 32 + b.units - 1) / b.units);  // of one block
+    const int rows = rows_that_fit(bits, f32 ? 3 : 1, K, w->G, (int)(M < 16 ? M : 16));
+    const int64_t tiles = (w->N + qmm::kTile - 1) / qmm::kTile, per_block = tiles_per_chunk(tiles, cus);
+    // qmm's blocks, each counted by the tiles its waves work through
+    const int64_t blocks = (M + rows - 1) / rows * ((tiles + per_block - 1) / per_block) * (per_block / qmm::kWaves);
+    if (qmm::straight_line(bits, K, w->G, f32, rows)) {
+        if (f32 && K <= 512) return true;
+        if (K <= 2048 && blocks <= std::min<int64_t>(f32 ? 4 : 3, 4096 / K) * cus) return true;
+        return !f32 && blocks <= cus && reg_rounds > cus;
+    }
+    const int64_t held = (int64_t)b.slices * b.spans * b.units;  // spans of x in a block's registers
+    if (held <= 16 || (f32 && held * span <= 2048)) return false;  // K = 256: little x (q4 5120 x 256 M = 24 6.8 / 6.2)
+    if (!f32) return K < 1024 && 2 * held > 9 * nspan && blocks <= (held * span > 4096 ? 2 : 1) * cus;
+    if (reg_tiles > cus / 8 && reg_rounds > cus &&
+        ((K <= 512 && blocks <= 3 * cus) || (K > 1024 && K <= 1280 && blocks <= 2 * cus)))
+        return true;
+    if (K >= 1024) return M == 1 && K <= 1280 && blocks <= cus;
+    if (80 * held <= (320 + (reg_rounds > cus ? 4 : bits == 4 ? 7 : 10) * rows) * nspan) return false;
+    return blocks <= 2 * cus || 2 * b.slices * b.spans >= 3 * nspan;
+}
+
 // Which kernel takes a dense linear. Up to 16 rows with a power of two of spans: dense_ks. Otherwise the register tiles
 // where they take the shape (reg_tiles.hpp), against
 //   - the 64-token tiles (from dense_min_tokens tokens): above kDenseSplitMaxTokens tokens those; up to there by the two
@@ -83,14 +127,9 @@ enum Kernel { kKSplit, kRegTiles, kWideTiles, kQmm };
 //     4096, q8 9 and 4.6), with a fifth in gs_kernel's favour. Both sides measured, register tiles / gs_kernel: q4 4096
 //     x 4096 M = 128 16.2 / 20.4 us, M = 200 26.5 / 21.2; 12288 x 4096 M = 400 98.9 / 120.1; 8192 x 2560 M = 128 18.8 /
 //     15.2; q8 4096 x 4096 M = 48 16.9 / 26.0, 12288 x 4096 M = 64 34.2 / 28.0;
-//   - qmm at short K, where a tile's activations outweigh its weights, and few products (qmm / register tiles: q4 2560 x
-//     640 M = 64 7.9 / 10.7 us, M = 200 12.0 / 11.0; 4096 x 1024 M = 48 7.4 / 9.2, M = 128 10.4 / 9.5; q8 5120 x 2048 M =
-//     18 9.3 / 11.5, 10752 x 2048 M = 36 14.4 / 17.5, 14000 x 2048 M = 40 26.9 / 21.6, where K = 2560 is not on qmm's
-//     straight-line path: 7680 x 2560 M = 24 29.3 / 13.9; FP32 rows, 4096 x 1024 M = 128 21.3 / 23.5, M = 300 41.4 / 31.3,
-//     q8 1296 x 2048 M = 68 18.7 / 26.2).
-Kernel dense_kernel(int bits, const sx_qview *w, int64_t M, int act, int out_act) {
+//   - qmm at short K (qmm_is_faster).
+Kernel dense_kernel(int bits, const sx_qview *w, int64_t M, int act, int out_act, int cus) {
     const int64_t N = w->N, K = w->K;
-    const int cus = device_cus();
     if (dks::eligible(bits, w->G, N, K, M, act, out_act, cus)) return kKSplit;
     const bool wide = M >= gg::dense_min_tokens(bits) && gg::eligible_dense(bits, w->G, K, act) && aligned(w->scale, 4) &&
                       aligned(w->minv, 4);
@@ -104,13 +143,7 @@ Kernel dense_kernel(int bits, const sx_qview *w, int64_t M, int act, int out_act
         const double split = waves * (bits == 4 ? 6 + 15 * k : 4 + 23 * k);
         return reg * 1.2 < split ? kRegTiles : kWideTiles;
     }
-    const double macs = (double)M * (double)N * (double)K;
-    bool few;
-    if (act == SX_ACT_F32)
-        few = (bits == 4 ? K <= 1024 : K == 1024) ? macs < 6e8 : bits == 8 && K == 2048 && macs < 4e8;
-    else
-        few = bits == 4 ? K <= 1024 && macs < 3.5e8 : (K == 1024 || K == 2048) && macs < 9e8;
-    return few ? kQmm : kRegTiles;
+    return qmm_is_faster(bits, w, M, act, cus) ? kQmm : kRegTiles;
 }
 
 int linear(const char *fn, int bits, const void *x, const sx_qview *w, void *y, int64_t M, int act, int out_act,
@@ -124,7 +157,7 @@ int linear(const char *fn, int bits, const void *x, const sx_qview *w, void *y, 
              " with input ", act, " unsupported (same dtype, or BF16 -> F32)");
     SX_CHECK(apart(x, M * w->K * act_bytes(act), y, M * w->N * act_bytes(out_act)), fn, " output y [", y, ", +",
              M * w->N * act_bytes(out_act), " B) overlaps input x [", x, ", +", M * w->K * act_bytes(act), " B)");
-    switch (dense_kernel(bits, w, M, act, out_act)) {
+    switch (dense_kernel(bits, w, M, act, out_act, device_cus())) {
     case kKSplit: {  // decode width: K split over a block
         dks::Params d{};
         d.x = x, d.q = w->q, d.scale = w->scale, d.minv = w->minv, d.y = y, d.M = (int)M, d.N = w->N, d.K = w->K;
@@ -200,6 +233,21 @@ int sx_linear_q4(const void *x, const sx_qview *w, void *y, int64_t M, int act, 
 
 int sx_linear_q8(const void *x, const sx_qview *w, void *y, int64_t M, int act, int out_act, sx_stream stream) {
     return linear("sx_linear_q8", 8, x, w, y, M, act, out_act, stream);
+}
+
+const char *sx_linear_kernel(const sx_qview *w, int bits, int64_t M, int act, int out_act, int cus) {
+    const char *fn = "sx_linear_kernel";
+    if (!(bits == 4 || bits == 8) || M < 1) {
+        set_error(cat(fn, ": bits = ", bits, " (4 or 8), M = ", M, " (>= 1)"));
+        return nullptr;
+    }
+    if (check_view(fn, w, bits)) return nullptr;
+    switch (dense_kernel(bits, w, M, act, out_act, cus > 0 ? cus : device_cus())) {
+    case kKSplit: return "k_split";
+    case kRegTiles: return "register_tiles";
+    case kWideTiles: return M > gg::kDenseSplitMaxTokens ? "wide_tiles" : "wide_tiles_k_split";
+    default: return "qmm";
+    }
 }
 
 int sx_mtp_head_pick(const void *x, const sx_qview *w, int bits, float *logits, const uint32_t *router_err,

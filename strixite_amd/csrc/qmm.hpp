@@ -24,6 +24,8 @@ constexpr int kWaves = 4;
 constexpr int kThreads = kWaves * 64;
 constexpr int kTile = 16;     // weight rows per MFMA tile = activation rows per pass
 constexpr int kSpanBytes = 64;
+constexpr int kPrefetch = 8;  // steps (16-byte loads a lane) a group
+constexpr int stage_chunks(bool f32) { return f32 ? 4 : 12; }  // 8-element chunks of x a thread stages in one round
 
 enum Mode {
     DENSE = 0,         // y[m, n] = x[m] . W[n]                          (linear_q4 / linear_q8)
@@ -62,6 +64,14 @@ inline size_t lds_bytes(int bits, int nsplit, int64_t K, int64_t G, int rows, in
     const int64_t run = G < span_codes ? G : span_codes;
     const int64_t runs = (K + span_codes - 1) / span_codes * (span_codes / run);
     return (size_t)nsplit * rows * (K + 8) * 2 + (size_t)blocks * runs * 16 * 4 + 2048;
+}
+
+// Whether a launch of `rows` staged rows takes the kernel's straight-line path (one staging round, whole groups of steps,
+// a span one quantization group); SWIGLU modes take it from half that K too.
+inline bool straight_line(int bits, int64_t K, int64_t G, bool f32, int rows) {
+    const int64_t span_codes = bits == 4 ? 128 : 64;
+    return G == span_codes && K % (span_codes * kPrefetch) == 0 && (K & (K - 1)) == 0 &&
+           rows * (K / 8) <= kThreads * stage_chunks(f32);
 }
 
 // Launches one mode; bits 4 / 8, act of x and y, nsplit 1 (BF16 x) or 3 (F32 x). grid.x = units * nchunks,

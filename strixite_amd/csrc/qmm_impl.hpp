@@ -11,7 +11,6 @@ namespace detail {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kPrefetch = 8;  // steps (16-byte loads a lane) a group
 constexpr int kRing = 1;      // groups in flight a wave (fast path)
 constexpr int kStageLoads = 8;  // activation chunk loads in flight a thread while staging
 constexpr int kZeroBytes = 2048;  // zero A operand for a group of idle-lane reads (8 q4 spans of BF16)
@@ -399,7 +398,7 @@ __global__ void __launch_bounds__(kThreads) qmm_kernel(Params p) {
         }
     };
 
-    constexpr int kStageMax = sizeof(TX) == 4 ? 4 : 12;  // chunks a thread the fast path stages in one round
+    constexpr int kStageMax = stage_chunks(sizeof(TX) == 4);  // chunks a thread the fast path stages in one round
     if (fast && T_all <= cap && (MODE == SLOT_COMBINE ? R : T_all) * chunks8 <= kThreads * kStageMax &&
         (chunks8 & (chunks8 - 1)) == 0) {
         // One batch, one staging round, straight-line: the activation loads go out first, then the weight loads of

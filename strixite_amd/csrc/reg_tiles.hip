@@ -66,6 +66,12 @@ bool eligible_dense(int bits, int64_t G, int64_t N, int64_t K, int64_t M, int ac
     return N * (K * bits / 8) < (int64_t(1) << 32) && tiles * (N / 32 + 1) < (int64_t(1) << 31) && N < (1 << 27);
 }
 
+Block dense_block(int bits, int64_t K, int act) {
+    const detail::Split s = bits == 4 ? detail::kSplits4[detail::split_of((int)(K / 128), detail::kSplits4)]
+                                      : detail::kSplits8[detail::split_of((int)(K / 64), detail::kSplits8)];
+    return {s.q, s.spw, detail::lanes_of(bits, s.q, act == SX_ACT_F32)};
+}
+
 hipError_t launch_dense(int bits, const void *x, const sx_qview *w, void *y, int64_t M, int act, int out_act,
                         hipStream_t stream) {
     detail::Params p{};

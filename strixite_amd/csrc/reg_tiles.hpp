@@ -21,5 +21,10 @@ hipError_t launch_grouped(int mode, const void *x, const sx_qview *w, void *y, c
 bool eligible_dense(int bits, int64_t G, int64_t N, int64_t K, int64_t M, int act);
 hipError_t launch_dense(int bits, const void *x, const sx_qview *w, void *y, int64_t M, int act, int out_act,
                         hipStream_t stream);
+// A dense block (an eligible shape): K slices, spans a slice, output units (32 rows) it works on at once.
+struct Block {
+    int slices, spans, units;
+};
+Block dense_block(int bits, int64_t K, int act);
 
 }  // namespace sx::rt

@@ -33,7 +33,7 @@ namespace {
 
 using qmm::detail::bf16x8;
 using qmm::detail::f32x4;
-using qmm::detail::kPrefetch;
+using qmm::kPrefetch;
 
 constexpr int kThreads = 512, kWaves = 8;
 constexpr int kLag = 2;  // a slot's reload goes out two slots after its unpack (fewer loads in flight: measured faster)

@@ -127,3 +127,49 @@ def test_engine_draft_and_commit_rules():
     assert [commit_after_accept(j, 5) for j in range(5)] == [("keep_verify_prefix", j + 1) for j in range(5)]
     with pytest.raises(ValueError):
         commit_after_accept(6, 5)
+
+
+# ---------------- which kernel takes a dense linear (256 compute units) ----------------
+
+def linear_kernel(L, bits, M, N, K, act=sx.ACT_BF16, out_act=None, G=None, scale_at=0):
+    """sx_linear_kernel's answer for a view whose scales start scale_at bytes past a 16-byte boundary."""
+    base = 1 << 20
+    w = sx.QView(base, base + scale_at, base, N, K, G or (128 if bits == 4 else 64))
+    name = L.sx_linear_kernel(ctypes.byref(w), bits, M, act, act if out_act is None else out_act, 256)
+    return name.decode() if name else None
+
+
+@pytest.mark.parametrize("bits,act,M,N,K,kernel", [
+    # short K on qmm's straight-line path, every K that has it, up to 4096 / K blocks a compute unit
+    (8, sx.ACT_BF16, 24, 4096, 512, "qmm"), (8, sx.ACT_BF16, 37, 14000, 512, "qmm"),
+    (8, sx.ACT_BF16, 24, 14000, 1024, "qmm"), (8, sx.ACT_BF16, 24, 14000, 2048, "qmm"),
+    (8, sx.ACT_BF16, 32, 14000, 2048, "register_tiles"), (8, sx.ACT_BF16, 24, 8192, 4096, "register_tiles"),
+    (4, sx.ACT_BF16, 64, 8192, 1024, "qmm"), (4, sx.ACT_BF16, 95, 14000, 1024, "register_tiles"),
+    (4, sx.ACT_BF16, 24, 8192, 2048, "register_tiles"),  # 13 staged rows: past that path's one staging round
+    (8, sx.ACT_F32, 128, 14000, 512, "qmm"), (8, sx.ACT_F32, 37, 5120, 1024, "qmm"),
+    (4, sx.ACT_F32, 128, 14000, 1024, "register_tiles"),
+    # its general path, where a block of register tiles holds x several times over
+    (8, sx.ACT_BF16, 16, 8192, 768, "qmm"), (8, sx.ACT_BF16, 17, 14000, 768, "register_tiles"),
+    (8, sx.ACT_BF16, 24, 5120, 960, "register_tiles"), (8, sx.ACT_F32, 6, 14000, 768, "qmm"),
+    (8, sx.ACT_F32, 37, 14000, 768, "register_tiles"), (8, sx.ACT_F32, 200, 5120, 320, "qmm"),
+    (4, sx.ACT_BF16, 37, 5120, 640, "qmm"), (4, sx.ACT_BF16, 300, 5120, 640, "register_tiles"),
+    (4, sx.ACT_BF16, 24, 5120, 256, "register_tiles"), (4, sx.ACT_F32, 6, 8192, 896, "qmm"),
+    (4, sx.ACT_F32, 17, 8192, 896, "register_tiles"),
+    # FP32 rows in many 5-token tiles of few rows
+    (4, sx.ACT_F32, 200, 1000, 1152, "qmm"), (4, sx.ACT_F32, 128, 1000, 1152, "register_tiles"),
+    # longer K
+    (8, sx.ACT_BF16, 6, 300, 1152, "register_tiles"), (4, sx.ACT_F32, 6, 5120, 2560, "register_tiles"),
+])
+def test_short_k_linears_keep_the_faster_kernel(L, bits, act, M, N, K, kernel):
+    """The register tiles against qmm at short K: q8 K = 512 and 768 and q4 K = 1024 at 4e8 .. 9e8 products ran up to 2.2
+    times as long on the register tiles, FP32 rows up to 2.1 times."""
+    assert linear_kernel(L, bits, M, N, K, act) == kernel
+
+
+def test_linear_kernel_names(L):
+    assert linear_kernel(L, 4, 1, 4096, 4096, sx.ACT_F32) == "k_split"
+    assert linear_kernel(L, 4, 200, 4096, 4096) == "wide_tiles_k_split"
+    assert linear_kernel(L, 4, 513, 4096, 4096) == "wide_tiles"
+    assert linear_kernel(L, 4, 200, 4096, 4096, scale_at=2) == "register_tiles"  # the wide tiles read scales in pairs
+    assert linear_kernel(L, 4, 24, 4096, 4096, G=64) == "qmm"
+    assert linear_kernel(L, 4, 0, 4096, 4096) is None and b"M = 0" in L.sx_last_error()
