@@ -52,6 +52,8 @@ int sx_linear_q8(const void *x, const sx_qview *w, void *y, int64_t M, int act, 
  * "register_tiles", "wide_tiles_k_split", "wide_tiles" or "qmm"; NULL for a view or width no call takes (sx_last_error).
  * For tests and profiles; no reference counterpart. */
 const char *sx_linear_kernel(const sx_qview *w, int bits, int64_t M, int act, int out_act, int cus);
+/* The same for the grouped expert calls (gather, its SwiGLU form, combine): "register_tiles", "wide_tiles" or "qmm". */
+const char *sx_experts_grouped_kernel(const sx_qview *w, int64_t E, int64_t M, int64_t A, int act, int cus);
 
 /* ---- per-slot MoE experts (decode / short verify), kernels/linear_q4.hpp:32-58 ----
  * w: E experts stacked [E*N, K]; ids [M, A] int32 device. err: >= 3 zeroed uint32 (device).

@@ -65,6 +65,7 @@ SIGNATURES = {
     "sx_linear_q4": [_P, _QV, _P, _I64, _INT, _INT, _P],
     "sx_linear_q8": [_P, _QV, _P, _I64, _INT, _INT, _P],
     "sx_linear_kernel": [_QV, _INT, _I64, _INT, _INT, _INT],
+    "sx_experts_grouped_kernel": [_QV, _I64, _I64, _I64, _INT, _INT],
     "sx_linear_q4_experts_gather": [_P, _QV, _I64, _P, _I64, _I64, _P, _INT, _P, _P],
     "sx_linear_q4_experts_gather_swiglu": [_P, _QV, _I64, _P, _I64, _I64, _P, _INT, _P, _P],
     "sx_linear_q4_experts_combine": [_P, _QV, _I64, _P, _P, _I64, _I64, _P, _INT, _P, _P],
@@ -122,7 +123,7 @@ SIGNATURES = {
     "sx_probe_mfma": [_INT, _INT, _P, ctypes.POINTER(_D), _P],
 }
 _RESTYPES = {"sx_last_error": ctypes.c_char_p, "sx_version": ctypes.c_char_p, "sx_linear_kernel": ctypes.c_char_p,
-             "sx_strix_hash64": _U64, "sx_strixw_close": None}
+             "sx_experts_grouped_kernel": ctypes.c_char_p, "sx_strix_hash64": _U64, "sx_strixw_close": None}
 
 _lib = None
 

@@ -211,13 +211,33 @@ int grouped_common(const char *fn, const void *x, const sx_qview *w, int64_t E, 
 
 // Which kernel takes a grouped call: the 64-slot tiles from kPrefillMinTokens tokens and more than kMaxSlotsAnExpert
 // slots an expert on average, the register tiles otherwise (and where the 64-slot ones do not take the shape), qmm for
-// the rest (other group sizes, FP32 activations, long K).
-Kernel grouped_kernel(const sx_qview *w, int64_t M, int64_t A, int64_t E, int act) {
+// the rest (other group sizes, FP32 activations, long K) and, below kPrefillMinTokens tokens, on its straight-line path
+// with few weight tiles (16 rows of one slot tile) a compute unit: K = 1024 up to 21; K = 2048, where the register tiles
+// are the faster ones while every block is alone on its compute unit (up to 4), 4 to 9. Measured, qmm / register tiles in
+// us (weight tiles a compute unit): down, E = 8 4096 x 1024 A = 2 M = 2 (4) 8.5 / 10.2, M = 24 (13) 11.9 / 16.1; E = 32 2048 x
+// 1024 A = 4 M = 31 (20.5) 16.6 / 17.0; E = 512 4096 x 1024 A = 10 M = 2 (20) 18.4 / 21.4, M = 4 (40) 31.1 / 25.7, M = 12 (120)
+// 61.0 / 48.9; gate_up, E = 128 d = 2048 I = 768 A = 8 M = 1 (3) 9.6 / 8.2, M = 2 (6) 10.0 / 11.6, M = 4 (12) 16.5 / 14.5; E = 64
+// d = 2048 I = 512 A = 8 M = 4 (8) 11.4 / 12.1.
+// The rule looks at the weight's rows alone, so that a gather and its SwiGLU form run the same kernel (the same bits).
+Kernel grouped_kernel(const sx_qview *w, int64_t M, int64_t A, int64_t E, int act, int cus) {
     const bool wide = M >= gg::kPrefillMinTokens && gg::eligible(4, w->G, w->K, act) && aligned(w->scale, 4) &&
                       aligned(w->minv, 4);
-    const bool reg = rt::eligible_grouped(4, w->G, w->N / E, w->K, M, A, E, act);
-    if (reg && !(wide && M * A > rt::kMaxSlotsAnExpert * E)) return kRegTiles;
-    return wide ? kWideTiles : kQmm;
+    if (!rt::eligible_grouped(4, w->G, w->N / E, w->K, M, A, E, act)) return wide ? kWideTiles : kQmm;
+    if (wide && M * A > rt::kMaxSlotsAnExpert * E) return kWideTiles;
+    const int64_t S = M * A, slot_tiles = std::min(S, S / 16 + E + 2);
+    const int64_t tiles = slot_tiles * ((w->N / E + qmm::kTile - 1) / qmm::kTile);
+    const bool few = w->K <= 1024 ? tiles <= 21 * cus : w->K <= 2048 && tiles > 4 * cus && tiles <= 9 * cus;
+    if (M < gg::kPrefillMinTokens && few && qmm::straight_line(4, w->K, w->G, false, 12)) return kQmm;
+    return kRegTiles;
+}
+
+const char *kernel_name(Kernel k, bool k_split) {
+    switch (k) {
+    case kKSplit: return "k_split";
+    case kRegTiles: return "register_tiles";
+    case kWideTiles: return k_split ? "wide_tiles_k_split" : "wide_tiles";
+    default: return "qmm";
+    }
 }
 
 }  // namespace
@@ -242,12 +262,18 @@ const char *sx_linear_kernel(const sx_qview *w, int bits, int64_t M, int act, in
         return nullptr;
     }
     if (check_view(fn, w, bits)) return nullptr;
-    switch (dense_kernel(bits, w, M, act, out_act, cus > 0 ? cus : device_cus())) {
-    case kKSplit: return "k_split";
-    case kRegTiles: return "register_tiles";
-    case kWideTiles: return M > gg::kDenseSplitMaxTokens ? "wide_tiles" : "wide_tiles_k_split";
-    default: return "qmm";
+    return kernel_name(dense_kernel(bits, w, M, act, out_act, cus > 0 ? cus : device_cus()),
+                       M <= gg::kDenseSplitMaxTokens);
+}
+
+const char *sx_experts_grouped_kernel(const sx_qview *w, int64_t E, int64_t M, int64_t A, int act, int cus) {
+    const char *fn = "sx_experts_grouped_kernel";
+    if (check_view(fn, w, 4)) return nullptr;
+    if (!(E >= 1 && w->N % E == 0 && M >= 1 && A >= 1 && A <= E)) {
+        set_error(cat(fn, ": E = ", E, " of ", w->N, " rows, M = ", M, ", A = ", A));
+        return nullptr;
     }
+    return kernel_name(grouped_kernel(w, M, A, E, act, cus > 0 ? cus : device_cus()), false);
 }
 
 int sx_mtp_head_pick(const void *x, const sx_qview *w, int bits, float *logits, const uint32_t *router_err,
@@ -327,7 +353,7 @@ int sx_linear_q4_experts_gather_grouped(const void *x, const sx_qview *w, int64_
     if (int rc = grouped_common(fn, x, w, E, M, A, ws, ws_bytes, y, act, math)) return rc;
     const int64_t N = w->N / E, es = act_bytes(act), S = M * A;
     SX_CHECK(apart(x, M * w->K * es, y, S * N * es), fn, " y overlaps x");
-    const Kernel kernel = grouped_kernel(w, M, A, E, act);
+    const Kernel kernel = grouped_kernel(w, M, A, E, act, device_cus());
     const int32_t *route = static_cast<const int32_t *>(ws);
     if (kernel != kQmm) {
         SX_HIP(kernel == kRegTiles ? rt::launch_grouped(qmm::GATHER, x, w, y, route, M, A, E, stream_of(stream))
@@ -350,7 +376,7 @@ int sx_linear_q4_experts_gather_swiglu_grouped(const void *x, const sx_qview *w,
     const int64_t N = w->N / E, es = act_bytes(act), S = M * A;
     SX_CHECK(N % 2 == 0, fn, " SwiGLU gather needs an even row count per expert ([gate | up]), got ", N);
     SX_CHECK(apart(x, M * w->K * es, h, S * (N / 2) * es), fn, " h overlaps x");
-    const Kernel kernel = grouped_kernel(w, M, A, E, act);
+    const Kernel kernel = grouped_kernel(w, M, A, E, act, device_cus());
     const int32_t *route = static_cast<const int32_t *>(ws);
     if (kernel != kQmm) {
         SX_HIP(kernel == kRegTiles ? rt::launch_grouped(qmm::SWIGLU, x, w, h, route, M, A, E, stream_of(stream))
@@ -376,7 +402,7 @@ int sx_linear_q4_experts_combine_grouped(const void *h, const sx_qview *w, int64
     SX_CHECK(apart(y, M * N * es, h, S * w->K * es), fn, " y overlaps h");
     SX_CHECK(apart(y, M * N * es, partial, S * N * 4), fn, " y overlaps partial");
     SX_CHECK(apart(partial, S * N * 4, h, S * w->K * es), fn, " partial overlaps h");
-    const Kernel kernel = grouped_kernel(w, M, A, E, act);
+    const Kernel kernel = grouped_kernel(w, M, A, E, act, device_cus());
     const int32_t *route = static_cast<const int32_t *>(ws);
     if (kernel != kQmm) {
         SX_HIP(kernel == kRegTiles ? rt::launch_grouped(qmm::COMBINE, h, w, partial, route, M, A, E, stream_of(stream))

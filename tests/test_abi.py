@@ -173,3 +173,21 @@ def test_linear_kernel_names(L):
     assert linear_kernel(L, 4, 200, 4096, 4096, scale_at=2) == "register_tiles"  # the wide tiles read scales in pairs
     assert linear_kernel(L, 4, 24, 4096, 4096, G=64) == "qmm"
     assert linear_kernel(L, 4, 0, 4096, 4096) is None and b"M = 0" in L.sx_last_error()
+
+
+# ---------------- which kernel takes a grouped expert call ----------------
+
+@pytest.mark.parametrize("E,rows,K,A,M,kernel", [
+    (8, 4096, 1024, 2, 1, "qmm"), (8, 4096, 1024, 2, 31, "qmm"),          # a down projection, short K
+    (8, 4096, 1024, 2, 32, "register_tiles"),                             # against the 64-slot tiles from here on
+    (32, 2048, 1024, 4, 31, "qmm"), (512, 4096, 1024, 10, 2, "qmm"), (512, 4096, 1024, 10, 4, "register_tiles"),
+    (16, 7168, 1024, 4, 2, "qmm"), (16, 7168, 1024, 4, 4, "register_tiles"),
+    (128, 1536, 2048, 8, 1, "register_tiles"), (128, 1536, 2048, 8, 2, "qmm"), (128, 1536, 2048, 8, 4, "register_tiles"),
+    (64, 2048, 512, 8, 2, "register_tiles"), (513, 2560, 640, 11, 6, "register_tiles"),
+    (512, 2048, 4096, 10, 1, "register_tiles"),                           # a gate_up projection, long K
+    (512, 2048, 4096, 10, 716, "register_tiles"), (512, 2048, 4096, 10, 717, "wide_tiles"),  # 14 slots an expert
+])
+def test_grouped_calls_keep_the_faster_kernel(L, E, rows, K, A, M, kernel):
+    """Few slot tiles at short K ran up to 1.8 times as long on the register tiles as on qmm."""
+    w = sx.QView(1 << 20, 1 << 20, 1 << 20, E * rows, K, 128)
+    assert L.sx_experts_grouped_kernel(ctypes.byref(w), E, M, A, sx.ACT_BF16, 256).decode() == kernel
