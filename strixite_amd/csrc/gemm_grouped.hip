@@ -1276,7 +1276,7 @@ __device__ __forceinline__ void gw_run(const Params &p, unsigned char *x0, unsig
     if constexpr (sizeof(TY) == 2) {
         if (p.vec_store) {  // BF16 through LDS (every wave is past its K loop and has drained its DMA: the barrier)
             constexpr int kRowB = 32 * 2, kChunksRow = 4, kWaveB = kBM * kRowB;  // 8 KB a wave
-            static_assert(2 * kWaveB <= kStageBytes, "two waves' staged outputs fit a stage array");
+            static_assert(2 * kWaveB <= W::kStageBytes, "two waves' staged outputs fit a stage array");
             asm volatile("s_barrier" ::: "memory");
             unsigned char *stg = xs_at(wave >> 1) + (wave & 1) * kWaveB;
 #pragma unroll
