@@ -357,7 +357,7 @@ int sx_linear_q4_experts_gather_grouped(const void *x, const sx_qview *w, int64_
     const int32_t *route = static_cast<const int32_t *>(ws);
     if (kernel != kQmm) {
         SX_HIP(kernel == kRegTiles ? rt::launch_grouped(qmm::GATHER, x, w, y, route, M, A, E, stream_of(stream))
-                                   : gg::launch(qmm::GATHER, x, w, y, route, M, A, E, act, stream_of(stream)), fn);
+                                   : gg::launch(qmm::GATHER, x, w, y, route, M, A, E, stream_of(stream)), fn);
         return SX_OK;
     }
     Params p{};
@@ -380,7 +380,7 @@ int sx_linear_q4_experts_gather_swiglu_grouped(const void *x, const sx_qview *w,
     const int32_t *route = static_cast<const int32_t *>(ws);
     if (kernel != kQmm) {
         SX_HIP(kernel == kRegTiles ? rt::launch_grouped(qmm::SWIGLU, x, w, h, route, M, A, E, stream_of(stream))
-                                   : gg::launch(qmm::SWIGLU, x, w, h, route, M, A, E, act, stream_of(stream)), fn);
+                                   : gg::launch(qmm::SWIGLU, x, w, h, route, M, A, E, stream_of(stream)), fn);
         return SX_OK;
     }
     Params p{};
@@ -406,7 +406,7 @@ int sx_linear_q4_experts_combine_grouped(const void *h, const sx_qview *w, int64
     const int32_t *route = static_cast<const int32_t *>(ws);
     if (kernel != kQmm) {
         SX_HIP(kernel == kRegTiles ? rt::launch_grouped(qmm::COMBINE, h, w, partial, route, M, A, E, stream_of(stream))
-                                   : gg::launch(qmm::COMBINE, h, w, partial, route, M, A, E, SX_ACT_F32, stream_of(stream)), fn);
+                                   : gg::launch(qmm::COMBINE, h, w, partial, route, M, A, E, stream_of(stream)), fn);
         return combine_reduce(partial, ids, coef, M, A, E, N, y, act, stream_of(stream));
     }
     Params p{};

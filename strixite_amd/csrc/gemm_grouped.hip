@@ -353,9 +353,9 @@ __global__ void __launch_bounds__(kThreads, 2) gg_kernel(Params p) {
     //   at the top of step k, the pair issued at the top of step k - 2 has landed (with 10, the two more of the steps
     //   that issue a window, the last two DMA instructions - four rows each - of the steps that issue none could
     //   still be in flight: four slots of a tile wrong now and then on a cold run). What may still be out are
-    //   register loads, which the compiler waits for before their first use. A wave with no DMA (!dma_on) has no pair to wait for; the same
-    //   count only waits for older register loads. The DMA of other waves is covered by their own wait before the
-    //   same barrier.
+    //   register loads, which the compiler waits for before their first use. A wave with no DMA (!dma_on) has no pair to
+    //   wait for; the same count only waits for older register loads. The DMA of other waves is covered by their own
+    //   wait before the same barrier.
     // A change to what a step issues, or to the order, changes these counts: re-derive them, and run the
     // grouped kernels twice on the same inputs (the parity tests do) - a load landing after its use shows up as
     // run-to-run differences.
@@ -1385,7 +1385,7 @@ bool eligible_dense(int bits, int64_t G, int64_t K, int act) {
 }
 
 hipError_t launch(int mode, const void *x, const sx_qview *w, void *y, const int32_t *ws, int64_t M, int64_t A,
-                  int64_t E, int out_act, hipStream_t stream) {
+                  int64_t E, hipStream_t stream) {
     Params p{};
     p.x = static_cast<const uint16_t *>(x), p.q = static_cast<const uint8_t *>(w->q);
     p.scale = static_cast<const uint16_t *>(w->scale), p.minv = static_cast<const uint16_t *>(w->minv);
@@ -1393,17 +1393,17 @@ hipError_t launch(int mode, const void *x, const sx_qview *w, void *y, const int
     const int64_t S = M * A;
     const int64_t wtiles = S / kBM + E + 2;  // WTmax: an upper bound of the 64-slot tiles; the rest exit at once
     const int64_t out_rows = mode == qmm::SWIGLU ? p.N / 2 : p.N;
-    p.vec_store = out_act == SX_ACT_BF16 && out_rows % 8 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
+    p.vec_store = mode != qmm::COMBINE && out_rows % 8 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
     const int64_t per_block = mode == qmm::SWIGLU ? kWaves * 32 : kWaves * 64;
     p.nrb = (int)((out_rows + per_block - 1) / per_block);
     const dim3 grid((unsigned)((wtiles + 7) / 8 * 8 * p.nrb));
     hipError_t e;
     switch (mode) {
     case qmm::SWIGLU:
-        e = out_act == SX_ACT_F32 ? go<qmm::SWIGLU, float>(p, grid, stream) : go<qmm::SWIGLU, uint16_t>(p, grid, stream);
+        e = go<qmm::SWIGLU, uint16_t>(p, grid, stream);
         break;
     case qmm::GATHER:
-        e = out_act == SX_ACT_F32 ? go<qmm::GATHER, float>(p, grid, stream) : go<qmm::GATHER, uint16_t>(p, grid, stream);
+        e = go<qmm::GATHER, uint16_t>(p, grid, stream);
         break;
     default:
         if (p.K <= kPdMaxSteps * kSpan && (p.K / kSpan == 8 || p.K / kSpan == 4)) {  // the down projection

@@ -22,11 +22,12 @@ constexpr int64_t dense_min_tokens(int bits) { return bits == 8 ? kDenseMinToken
 constexpr int64_t kDenseSplitMaxTokens = 512;
 // The dense linears the tiles take: eligible's q4, and q8 (G = 64, K % 256 == 0, K <= 4096, BF16 x).
 bool eligible_dense(int bits, int64_t G, int64_t K, int act);
-// A dense linear at prefill width on the same tiles: y [M, w->N] (BF16 or FP32) = x [M, K] (BF16) . deq(w)^T, tile u
-// = tokens 64 u .. 64 u + 63 (eligible_dense(bits, G, K, BF16)).
+// A dense linear at prefill width: y [M, w->N] (BF16 or FP32) = x [M, K] (BF16) . deq(w)^T (eligible_dense(bits, G, K,
+// BF16)), in gs_kernel's blocks of 64 tokens x 64 rows up to kDenseSplitMaxTokens tokens, above in gw_kernel's units of 128
+// tokens x 256 rows.
 hipError_t launch_dense(const void *x, const sx_qview *w, void *y, int64_t M, int out_act, hipStream_t stream);
-// mode: qmm::SWIGLU (h [S, N/2]), qmm::GATHER (y [S, N]), qmm::COMBINE (FP32 partials [S, N]); N = w->N / E.
+// mode: qmm::SWIGLU (h [S, N/2], BF16), qmm::GATHER (y [S, N], BF16), qmm::COMBINE (FP32 partials [S, N]); N = w->N / E.
 hipError_t launch(int mode, const void *x, const sx_qview *w, void *y, const int32_t *ws, int64_t M, int64_t A,
-                  int64_t E, int out_act, hipStream_t stream);
+                  int64_t E, hipStream_t stream);
 
 }  // namespace sx::gg
