@@ -8,7 +8,7 @@ import ctypes
 
 import torch
 
-from . import (ACT_BF16, ACT_F32, MOE_F32, LogitCand, MtpPick, QView, check, lib)
+from . import (ACT_BF16, ACT_F32, MOE_F32, SX_EINVAL, LogitCand, MtpPick, QView, SxError, check, lib)
 
 _c = ctypes.c_void_p
 
@@ -65,6 +65,23 @@ def linear(x, w, out_act=None, y=None, stream=None):
     f = lib().sx_linear_q4 if w.bits == 4 else lib().sx_linear_q8
     check(f(_p(x), w.view(), _p(y), M, act, out_act, _s(stream)))
     return y
+
+
+def linear_kernel(w, M, act=ACT_BF16, out_act=None):
+    """The kernel linear() runs for M rows of x against w: "k_split", "register_tiles", "wide_tiles_k_split",
+    "wide_tiles" or "qmm"."""
+    name = lib().sx_linear_kernel(w.view(), w.bits, M, act, act if out_act is None else out_act, 0)
+    if name is None:
+        raise SxError(SX_EINVAL, lib().sx_last_error().decode())
+    return name.decode()
+
+
+def experts_grouped_kernel(w, E, M, A, act=ACT_BF16):
+    """The kernel gather_grouped() and combine_grouped() run: "register_tiles", "wide_tiles" or "qmm"."""
+    name = lib().sx_experts_grouped_kernel(w.view(), E, M, A, act, 0)
+    if name is None:
+        raise SxError(SX_EINVAL, lib().sx_last_error().decode())
+    return name.decode()
 
 
 def _err(device):

@@ -84,16 +84,20 @@ def test_linear_k_not_a_whole_span(bits, K, G):
 
 @pytest.mark.parametrize("bits,act,out_act,M,N,K", [
     (4, orc.BF16, orc.F32, 1, 40, 2560),      # five slices; a partial pair of row tiles
-    (4, orc.BF16, orc.BF16, 17, 300, 384),    # three spans in one slice; one token in the second tile
+    (4, orc.BF16, orc.BF16, 17, 300, 256),    # two spans in one slice; one token in the second tile
+    (4, orc.BF16, orc.F32, 210, 1300, 384),   # three spans in one slice
+    (4, orc.BF16, orc.BF16, 60, 5000, 512),   # four spans in one slice
     (4, orc.BF16, orc.F32, 33, 1000, 2432),   # 19 spans: the last slice overlaps the one before
     (4, orc.BF16, orc.F32, 60, 5000, 2560),   # more units than blocks: whole blocks a tile
-    (4, orc.BF16, orc.BF16, 210, 700, 640),   # many tiles: blocks cross from one tile to the next
+    (4, orc.BF16, orc.BF16, 600, 2000, 640),  # five spans in one slice; more tiles than an eighth of the blocks: some
+                                              # cross from one tile to the next
+    (8, orc.BF16, orc.F32, 600, 1200, 320),   # the same, two slices of five spans (BF16 tiles of q8)
     (4, orc.F32, orc.F32, 5, 33, 4096),       # FP32 rows: exactly one tile of five tokens
     (4, orc.F32, orc.F32, 11, 520, 3584),     # a last tile of one token; seven slices
     (8, orc.BF16, orc.F32, 16, 100, 4096),    # eight slices of eight spans
     (8, orc.BF16, orc.BF16, 6, 4000, 2560),   # five slices, two units a round
     (8, orc.BF16, orc.F32, 37, 65, 640),      # ten spans in two slices of five
-    (8, orc.BF16, orc.F32, 20, 90, 320),      # five spans in two slices: overlap
+    (8, orc.BF16, orc.F32, 40, 6000, 320),    # five spans in two slices: overlap
     (8, orc.F32, orc.F32, 37, 300, 2560),
     (8, orc.F32, orc.F32, 4, 70, 1984),       # 31 spans
     (8, orc.F32, orc.F32, 130, 700, 1536),
@@ -105,10 +109,12 @@ def test_register_tiles_dense(bits, act, out_act, M, N, K):
     from strixite_amd import kernels as kx
     rng = np.random.default_rng(M + N + K + bits)
     w = util.rand_qweight(rng, bits, N, K, 128 if bits == 4 else 64)
+    wd = kx.QWeight.upload(w)
+    assert kx.linear_kernel(wd, M, act, out_act) == "register_tiles"
     x = rng.standard_normal((M, K)).astype(np.float32)
     x = x if act == orc.F32 else util.f32_to_bf16(x)
     print(f"register tiles q{bits} act={act} out={out_act} M={M} N={N} K={K}", flush=True)
-    y = kx.linear(util.f32_dev(x) if act == orc.F32 else util.bf16_dev(x), kx.QWeight.upload(w), out_act=out_act)
+    y = kx.linear(util.f32_dev(x) if act == orc.F32 else util.bf16_dev(x), wd, out_act=out_act)
     torch.cuda.synchronize()
     util.assert_close(util.host_bits(y), orc.linear_q(x, w, out_act=out_act), tol=1e-5 if out_act == orc.F32 else 1e-3,
                       what=f"register tiles q{bits} M={M} N={N} K={K}")
@@ -125,6 +131,7 @@ def test_register_tiles_dense(bits, act, out_act, M, N, K):
     (8, orc.BF16, 900, 2600, 512),    # q8 halves
 ])
 def test_prefill_units(bits, out_act, M, N, K):
-    """Dense linears above the K-split tiles' widths, at every way an XCD's last round of units is split."""
+    """Dense linears above the K-split tiles' widths, at every way an XCD's last round of units is split, against the
+    oracle (N not a multiple of 8 or FP32 out: one store a value)."""
     y, ref = run(bits, N, K, 128 if bits == 4 else 64, M, orc.BF16, out_act, seed=M + N)
     util.assert_close(y, ref, tol=1e-5 if out_act == orc.F32 else 1e-3, what=f"prefill units q{bits} M={M} N={N} K={K}")

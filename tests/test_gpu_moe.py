@@ -356,8 +356,9 @@ def test_grouped_layer_first_run_matches_repeats(M):
     from strixite_amd import synthetic as syn
     from strixite_amd.verify import MoeVerifyLayer
     E, d, I, k = 512, 4096, 1024, 10
-    layer = MoeVerifyLayer(syn.router_weight(E, d, seed=81), syn.qweight(4, E * 2 * I, d, 128, seed=82),
-                           syn.qweight(4, E * d, I, 128, seed=83), E, k, M)
+    gate_up, down = syn.qweight(4, E * 2 * I, d, 128, seed=82), syn.qweight(4, E * d, I, 128, seed=83)
+    assert kx().experts_grouped_kernel(gate_up, E, M, k) == kx().experts_grouped_kernel(down, E, M, k) == "wide_tiles"
+    layer = MoeVerifyLayer(syn.router_weight(E, d, seed=81), gate_up, down, E, k, M)
     x = syn.activations(M, d, seed=84)
     sync()
     print(f"grouped layer, first run against repeats, M={M}", flush=True)
@@ -397,6 +398,7 @@ def test_register_tiles_match_oracle(M, A, E, I, d):
     ids[M // 2, A - 1] = -1
     ids_d = torch.from_numpy(ids).cuda()
     Wgu = kx().QWeight.upload(wgu)
+    assert kx().experts_grouped_kernel(Wgu, E, M, A) == "register_tiles"
     xd = util.bf16_dev(x)
     print(f"register tiles M={M} A={A} E={E} I={I} d={d}", flush=True)
     ws, err = kx().group_routes(ids_d, E)
@@ -414,7 +416,9 @@ def test_register_tiles_match_oracle(M, A, E, I, d):
         return
     wdn = util.rand_qweight(rng, 4, E * 40, I, G)  # 40 output rows an expert: a partial pair of tiles
     coef = rng.random((M, A)).astype(np.float32)
-    y = kx().combine_grouped(h, kx().QWeight.upload(wdn), E, ids_d, util.f32_dev(coef), ws)
+    Wdn = kx().QWeight.upload(wdn)
+    assert kx().experts_grouped_kernel(Wdn, E, M, A) == ("register_tiles" if I > G else "qmm")  # one span: qmm
+    y = kx().combine_grouped(h, Wdn, E, ids_d, util.f32_dev(coef), ws)
     sync()
     ref_y, _ = orc.experts_combine(util.host_bits(h), wdn, E, ids, coef)
     util.assert_close(util.host_bits(y), ref_y, what="combine")

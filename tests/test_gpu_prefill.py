@@ -135,30 +135,26 @@ def test_config4_prefill_layer_full_size():
     util.assert_close(util.host_bits(y)[ytoks], ref_y, what="config 4 y (sampled tokens)")
 
 
-@pytest.mark.parametrize("bits,G,act,out_act,M,K", [(4, 128, orc.BF16, orc.BF16, 2048, 4096),
-                                                     (4, 128, orc.BF16, orc.F32, 2000, 2048),
-                                                     (4, 128, orc.BF16, orc.BF16, 257, 512),
-                                                     (8, 64, orc.BF16, orc.F32, 2048, 4096),
-                                                     (8, 64, orc.BF16, orc.BF16, 300, 1280),
-                                                     (8, 64, orc.BF16, orc.BF16, 256, 4352),
-                                                     (8, 64, orc.BF16, orc.F32, 200, 768),
-                                                     (4, 128, orc.F32, orc.F32, 2048, 4096),
-                                                     (4, 128, orc.BF16, orc.F32, 130, 1024),
-                                                     (4, 128, orc.BF16, orc.BF16, 512, 4096),
-                                                     (8, 64, orc.BF16, orc.BF16, 100, 2048),
-                                                     (8, 64, orc.BF16, orc.F32, 513, 256)])
-def test_dense_linear_prefill_width(bits, G, act, out_act, M, K):
-    """linear_q4 / linear_q8 at prefill width (the route *_wmma callers take; q4 G = 128 and q8 G = 64 with BF16 x on
-    the MFMA tiles: K split over a block's waves up to 512 tokens, whole K a block above; a partial last tile of tokens
-    and of rows included; K = 4352 past the tiles' limit on qmm) against the oracle."""
+@pytest.mark.parametrize("bits,G,act,out_act,M,K,kernel", [
+    (4, 128, orc.BF16, orc.BF16, 2048, 4096, "wide_tiles"), (4, 128, orc.BF16, orc.F32, 2000, 2048, "wide_tiles"),
+    (4, 128, orc.BF16, orc.BF16, 257, 512, "wide_tiles_k_split"), (8, 64, orc.BF16, orc.F32, 2048, 4096, "wide_tiles"),
+    (8, 64, orc.BF16, orc.BF16, 300, 1280, "wide_tiles_k_split"), (8, 64, orc.BF16, orc.BF16, 256, 4352, "qmm"),
+    (8, 64, orc.BF16, orc.F32, 200, 768, "wide_tiles_k_split"), (4, 128, orc.F32, orc.F32, 2048, 4096, "register_tiles"),
+    (4, 128, orc.BF16, orc.F32, 130, 1024, "register_tiles"), (4, 128, orc.BF16, orc.BF16, 512, 4096, "register_tiles"),
+    (8, 64, orc.BF16, orc.BF16, 100, 2048, "register_tiles"), (8, 64, orc.BF16, orc.F32, 513, 256, "wide_tiles")])
+def test_dense_linear_prefill_width(bits, G, act, out_act, M, K, kernel):
+    """linear_q4 / linear_q8 at prefill width (the route *_wmma callers take) on a weight of few rows, on each kernel that
+    takes such calls (K = 4352 past the tiles' limit), against the oracle."""
     N = 384
     rng = np.random.default_rng(bits * 10 + act)
     w = util.rand_qweight(rng, bits, N, K, G)
+    wd = kx().QWeight.upload(w)
+    assert kx().linear_kernel(wd, M, act, out_act) == kernel
     x = rng.standard_normal((M, K)).astype(np.float32)
     x = x if act == orc.F32 else util.f32_to_bf16(x)
     print(f"dense prefill q{bits} G{G} act={act} out={out_act}", flush=True)
     xd = util.f32_dev(x) if act == orc.F32 else util.bf16_dev(x)
-    y = kx().linear(xd, kx().QWeight.upload(w), out_act=out_act)
+    y = kx().linear(xd, wd, out_act=out_act)
     sync()
     ref = orc.linear_q(x, w, out_act=out_act)
     util.assert_close(util.host_bits(y), ref, what=f"dense q{bits} M={M}")
@@ -207,16 +203,18 @@ def test_dense_prefill_bench_shape(bits, G):
     util.assert_close(yh[:, feats], orc.linear_q(xh, fw), what=f"dense q{bits} (all tokens, 128 features)")
 
 
-@pytest.mark.parametrize("bits,G", [(4, 128), (8, 64)])
-def test_staged_stores_match_direct_stores(bits, G):
-    """The MFMA tiles store BF16 outputs through LDS as 16-byte vectors when y is 16-byte aligned (and the row count a
-    multiple of 8), and one value at a time otherwise: the two store paths write the same bits."""
+@pytest.mark.parametrize("bits,G,K", [(4, 128, 512), (8, 64, 256)])
+@pytest.mark.parametrize("M,N", [(600, 384), (700, 4096), (1024, 6144)])
+def test_staged_stores_match_direct_stores(bits, G, K, M, N):
+    """The 128-token units store BF16 outputs through LDS as 16-byte vectors when y is 16-byte aligned (and the row count
+    a multiple of 8), and one value at a time otherwise: the two store paths write the same bits. On 256 compute units
+    10, 96 and 192 units: an XCD's are done in quarters, in halves and whole."""
     import torch
-    M, N, K = 300, 384, 1024
     rng = np.random.default_rng(90 + bits)
     w = kx().QWeight.upload(util.rand_qweight(rng, bits, N, K, G))
+    assert kx().linear_kernel(w, M) == "wide_tiles"
     xd = util.bf16_dev(util.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32)))
-    print(f"staged vs direct stores q{bits}", flush=True)
+    print(f"staged vs direct stores q{bits} M={M} N={N}", flush=True)
     y = kx().linear(xd, w)
     buf = torch.empty(M * N + 1, dtype=torch.bfloat16, device="cuda")
     y2 = buf[1:].view(M, N)  # 2 bytes past a 16-byte boundary: the direct path
@@ -228,32 +226,41 @@ def test_staged_stores_match_direct_stores(bits, G):
 @pytest.mark.parametrize("bits,G,M,N,K,out_act", [(4, 128, 2048, 4096, 1024, orc.BF16), (8, 64, 2048, 4096, 512, orc.BF16),
                                                   (4, 128, 2000, 4104, 1024, orc.BF16), (8, 64, 2000, 4104, 512, orc.F32),
                                                   (4, 128, 2000, 4096, 512, orc.F32), (8, 64, 2048, 4100, 512, orc.BF16)])
-def test_wide_tiles_match_64_token_tiles(bits, G, M, N, K, out_act):
-    """Where its grid fills the chip (here: all M tokens at once) the dense linear takes 128 tokens a wave; each half
-    of the tokens alone takes gg_kernel's 64-token tiles. Both do the same arithmetic for every output: the same bits
-    (a partial last token tile, a partial last row block, BF16 staged and BF16 / F32 direct stores included)."""
-    import torch
+def test_whole_and_split_units_agree(bits, G, M, N, K, out_act):
+    """All M tokens at once and each half of them alone: on 256 compute units the 128-token units of one are whole where
+    the other's are split (4096 rows: whole against halves; 4104: whole rounds and quarters against whole). The same bits
+    (a partial last token tile, a partial last row block, BF16 staged and BF16 / F32 direct stores included), and 64
+    seeded tokens against the oracle."""
     rng = np.random.default_rng(M + N + K + bits)
-    w = kx().QWeight.upload(util.rand_qweight(rng, bits, N, K, G))
-    xd = util.bf16_dev(util.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32)))
-    print(f"wide vs 64-token tiles q{bits} M={M} N={N} K={K} out={out_act}", flush=True)
+    hw = util.rand_qweight(rng, bits, N, K, G)
+    w = kx().QWeight.upload(hw)
+    assert kx().linear_kernel(w, M, out_act=out_act) == kx().linear_kernel(w, M // 2, out_act=out_act) == "wide_tiles"
+    x = util.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32))
+    xd = util.bf16_dev(x)
+    print(f"whole and split units q{bits} M={M} N={N} K={K} out={out_act}", flush=True)
     y = kx().linear(xd, w, out_act=out_act)
     h = M // 2
     y0 = kx().linear(xd[:h].contiguous(), w, out_act=out_act)
     y1 = kx().linear(xd[h:].contiguous(), w, out_act=out_act)
     sync()
-    assert np.array_equal(util.host_bits(y), np.concatenate([util.host_bits(y0), util.host_bits(y1)]))
+    got = util.host_bits(y)
+    assert np.array_equal(got, np.concatenate([util.host_bits(y0), util.host_bits(y1)]))
+    toks = np.sort(rng.choice(M, 64, replace=False))
+    util.assert_close(got[toks], orc.linear_q(x[toks], hw, out_act=out_act), what=f"units q{bits} M={M} N={N}")
 
 
-@pytest.mark.parametrize("bits,G,M,N,K", [(4, 128, 100, 100, 512), (8, 64, 60, 72, 256), (4, 128, 511, 200, 1536),
-                                          (8, 64, 300, 40, 4096)])
+@pytest.mark.parametrize("bits,G,M,N,K", [(4, 128, 100, 100, 512), (8, 64, 60, 72, 256), (4, 128, 300, 1000, 1024),
+                                          (4, 128, 511, 1000, 1536), (4, 128, 500, 1210, 4096), (8, 64, 101, 1300, 2048),
+                                          (8, 64, 300, 900, 4096)])
 def test_dense_k_split_ragged(bits, G, M, N, K):
     """The K-split tiles (up to 512 tokens) on ragged shapes: output rows not a multiple of 64, one K step a wave
-    (K = 512 q4, 256 q8), a quarter of K not a multiple of the ring, against the oracle."""
+    (K = 512 q4, 256 q8), two, three and eight (q4), a quarter of K not a multiple of the ring, against the oracle."""
     rng = np.random.default_rng(M + N + K)
     w = util.rand_qweight(rng, bits, N, K, G)
+    wd = kx().QWeight.upload(w)
+    assert kx().linear_kernel(wd, M, out_act=orc.F32) == "wide_tiles_k_split"
     x = util.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32))
     print(f"dense k-split q{bits} M={M} N={N} K={K}", flush=True)
-    y = kx().linear(util.bf16_dev(x), kx().QWeight.upload(w), out_act=orc.F32)
+    y = kx().linear(util.bf16_dev(x), wd, out_act=orc.F32)
     sync()
     util.assert_close(util.host_bits(y), orc.linear_q(x, w, out_act=orc.F32), what=f"k-split q{bits} M={M} N={N}")
