@@ -1037,9 +1037,9 @@ __global__ void __launch_bounds__(kThreads, 1) gs_kernel(Params p) {
 // 81.8 -> 71.5 us, q8 117.9 -> 91.4 us.
 // The units are dealt to the XCDs in equal runs (all of a token tile on one XCD left the fifth to eighth XCD idle for
 // every token tile past a multiple of eight), and an XCD's last round, when at most half full, is split into 64- or
-// 32-token blocks (a step of a 64-token block takes 0.54 of a whole one's time): 7680 x 2560 q4 at M = 1531 93 -> 76
-// us, 9000 x 3072 M = 1300 159 -> 109, 4096 x 4096 M = 600 51.4 (gg_kernel) -> 41.9, 2560 x 2560 M = 520 33.2 ->
-// 21.5; q8 9000 x 2560 M = 1300 172 -> 119. What bounds a whole round: two waves a SIMD of MFMA and VALU work in
+// 32-token blocks (a step of a 64-token block takes 0.54 of a whole one's time): 7680 x 2560 q4 at M = 1531 95 -> 78
+// us (on another card 97 -> 82), 9000 x 3072 M = 1300 162 -> 113, 4096 x 4096 M = 600 54 (gg_kernel) -> 45, 2560 x 2560 M =
+// 520 35 -> 24; q8 9000 x 2560 M = 1300 176 -> 123. What bounds a whole round: two waves a SIMD of MFMA and VALU work in
 // turn, at a clock that the power limit holds near 2 GHz (8192 x 4096 M = 2048: 0.88 PFLOP/s, 1.02 with x all zero).
 constexpr int kGwThreads = 512, kGwWaves = 8, kGwBM = 128, kGwTB = kGwBM / 32, kGwRows = kGwWaves * 32;
 

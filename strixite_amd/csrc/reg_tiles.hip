@@ -1,6 +1,7 @@
 // Dequantizing GEMM with a tile's activations resident in registers: grouped experts with a few slots each (q4 G = 128,
 // BF16 x), from a handful of tokens to about 14 slots an expert; and dense linears (q4 G = 128, q8 G = 64, BF16 or FP32 x)
-// that dense_ks does not take: other K than a power of two of spans, 16 rows and more, up to prefill width.
+// that dense_ks does not take: other K than a power of two of spans, more than 16 rows, up to prefill width (short K stays
+// with qmm where that is the faster one: the rules are in api_qmm.hip).
 //
 // What bounds it: the experts' codes, read once a 16-slot tile; the work is weight streaming (4.7 - 5.4 TB/s of codes,
 // scales and mins against 6.35 for a plain streaming read; leaving out the dequant, the MFMAs or the SwiGLU changes no
@@ -27,9 +28,9 @@
 // (K = 640, qmm before): M = 200 136 -> 116, 2048 375 -> 338.
 // Dense: the tokens in tiles of 16 (FP32 rows: five tokens as three exact BF16 planes each, fifteen operand rows, so that
 // the K loop and its registers are the BF16 ones), the weight streamed once a tile, from the caches after the first.
-// Before (qmm) and after: q4 8192 x 2560 M = 24 18.8 -> 8.9 us, M = 64 35.6 -> 12.2; q8 2560 x 4096 FP32 rows M = 37 40.3 ->
-// 24, 7680 x 2560 FP32 rows M = 128 249 -> 93; the q8 head 248,320 x 2560 at M = 6 228 -> 136 (0.66 GB: 5.0 TB/s), 151,936 x
-// 4096 at M = 16 386 -> 129.
+// Before (qmm) and after, three weights in turn: q4 8192 x 2560 M = 24 19.5 -> 9.4 us, M = 64 36.8 -> 14.2; q8 2560 x 4096
+// FP32 rows M = 37 42.0 -> 23.9, 7680 x 2560 FP32 rows M = 128 247 -> 92; the q8 head 248,320 x 2560 at M = 6 228 -> 134 (0.68
+// GB: 5.1 TB/s), 151,936 x 4096 at M = 16 380 -> 129.
 #include "reg_tiles_impl.hpp"
 
 namespace sx::rt {

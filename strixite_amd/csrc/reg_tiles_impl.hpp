@@ -65,7 +65,11 @@ __device__ __forceinline__ float bf16_rounded(float v) { return (float)(__bf16)v
 __device__ __forceinline__ void put(float *y, int64_t i, float v) { y[i] = v; }
 __device__ __forceinline__ void put(uint16_t *y, int64_t i, float v) { y[i] = __builtin_bit_cast(uint16_t, (__bf16)v); }
 
-// Q K slices of SPW spans, P output units a round: blocks of Q P waves.
+// Q K slices of SPW spans, P output units a round: blocks of Q P waves. Eight waves where P can fill them up; past four
+// slices one unit, but two for q8's five (K = 2112 .. 2560, BF16 rows): five waves are two on one SIMD and one on each of
+// the others, ten are three or two on each. One unit / two, us: 248320 x 2560 M = 24 218 / 203, 248320 x 2112 M = 64 411 /
+// 332, 14000 x 2112 M = 200 80 / 68; where a block has a single round two cost more (4096 x 2560 M = 16 9.4 / 14.5, M = 1
+// 8.1 / 10.8; qmm 19.7 and 16.0).
 constexpr int lanes_of(int bits, int q, bool f32) { return q < 5 ? 8 / q : bits == 8 && q == 5 && !f32 ? 2 : 1; }  // P
 // Blocks a compute unit: two of at most 128 registers where the operands leave room (a wave's 512 codes of 16 rows are
 // 64 registers; q8 has twice the code and scale registers in flight, FP32 rows twice the loads), else one.
