@@ -1,8 +1,8 @@
-"""Benchmark of strixite's MTP verify path on one MI355X (BASELINE.json's metric).
+"""Benchmark of strixite's MTP verify path on one MI355X.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu] [--no-extra]
 
-A step is one MoE FFN verify sublayer: M = 6 tokens, hidden 4096, 512 experts, top-10 routing
+A step is one MoE FFN verify sublayer (config 3): M = 6 tokens, hidden 4096, 512 experts, top-10 routing
 from FP32 router logits, SwiGLU experts (gate_up [1024 x 2 x 4096], down [4096 x 1024]) in q4 G = 128. Each step takes
 the next of 16 distinct token batches (different routing each, so the 3.4 GB of experts are not served from the
 256 MB Infinity Cache), with every input resident in HBM before the timed region. One JSON line goes to stdout:
@@ -305,7 +305,7 @@ def cpu_baseline(layer, xs, budget_s, gpu_logits):
 
 
 def prefill_layer(steps=20, probe=False):
-    """x BF16 [2048, 4096] through the router projection, the Zipf bias, top-10 routing, grouping,
+    """Config 4: x BF16 [2048, 4096] through the router projection, the Zipf bias, top-10 routing, grouping,
     the grouped gate_up + SwiGLU and down + combine (q4 G = 128 experts, MFMA 64-slot x 128-row tiles)."""
     import torch
 

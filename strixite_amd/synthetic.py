@@ -1,6 +1,6 @@
 """Seeded synthetic inputs in the reference's formats, generated on the device (bench.py, smoke and the GPU tests).
 
-Weights follow BASELINE.json's configs with the reference's actual format (formats/q4.hpp:3-6, q8.hpp:3-11): uniform
+Weights are in the reference's actual format (formats/q4.hpp:3-6, q8.hpp:3-11): uniform
 codes, scale = bf16(|N(0, 0.02)|), min = bf16(-(2^bits - 1) / 2 * scale) so the weights are zero-mean. torch's
 device generator (Philox) makes them from the seed; the CPU oracle gets host copies of the same bytes.
 """
@@ -33,7 +33,7 @@ def router_weight(E, K, seed, device="cuda"):
 
 
 def zipf_router_bias(E, seed, s=1.1, scale=0.3, device="cuda"):
-    """BASELINE config 4's routing skew: a bias added to the router logits, -scale * s * ln(rank + 1) for the
+    """The prefill layer's routing skew: a bias added to the router logits, -scale * s * ln(rank + 1) for the
     experts in a seeded random order of ranks (a Zipf(s) prior in log space). scale = 0.3 against logits of standard
     deviation ~1.3 (x ~ N(0, 1), Wr ~ N(0, 0.02), d = 4096) gives buckets of 0..~450 of 20,480 slots at top-10."""
     g = torch.Generator().manual_seed(seed)

@@ -67,7 +67,7 @@ def check_against_oracle(x, Wr_host, wr_bf16, logits, ids, coef, h, y, gu, dn, E
 
 @pytest.mark.parametrize("wr_bf16", [False, True])
 def test_layer_config3_matches_oracle_and_two_launch(wr_bf16):
-    """BASELINE config 3 (M = 6, d = 4096, E = 512, top-10, I = 1024, q4 G = 128): FP32 router weight as the config
+    """Config 3 (M = 6, d = 4096, E = 512, top-10, I = 1024, q4 G = 128): FP32 router weight as the config
     states it, and the served model's BF16 weight."""
     import torch
     from strixite_amd import synthetic as syn

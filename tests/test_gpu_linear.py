@@ -40,14 +40,14 @@ def test_linear_dtypes_partial_tile(act, out_act, bits):
 
 
 def test_config1_dense_q4_gemv_f32():
-    # x fp32 [1 x 4096], W 4096 x 4096 q4 G = 128, y fp32
+    # Config 1: x fp32 [1 x 4096], W 4096 x 4096 q4 G = 128, y fp32
     got, ref = run(4, 4096, 4096, 128, 1, F32, F32, seed=0)
     util.assert_close(got, ref, what="config 1")
 
 
 @pytest.mark.parametrize("bits,G", [(4, 128), (8, 64)])
 def test_config2_verify_width(bits, G):
-    # x bf16 [6 x 4096], W 12288 x 4096, fp32 out
+    # Config 2: x bf16 [6 x 4096], W 12288 x 4096, fp32 out
     got, ref = run(bits, 12288, 4096, G, 6, BF16, F32, seed=1)
     util.assert_close(got, ref, what=f"config 2 q{bits}")
 

@@ -1,6 +1,6 @@
 """Parity of the MoE path on cuda:0 through the C ABI: router (kernels/moe_router.hpp), route grouping
 (kernels/moe_grouped.hpp:42-49), per-slot experts (kernels/linear_q4.hpp:32-58), grouped experts
-(kernels/moe_grouped.hpp:51-62), SwiGLU, and the full BASELINE config-3 layer against the CPU oracle."""
+(kernels/moe_grouped.hpp:51-62), SwiGLU, and the full verify layer (config 3) against the CPU oracle."""
 import numpy as np
 import pytest
 
@@ -277,7 +277,7 @@ def test_grouped_bad_id_rows_are_nan():
     assert torch.isnan(y[1]).all() and not torch.isnan(y[0]).any() and not torch.isnan(y[2]).any()
 
 
-# ---------------- BASELINE config 3 at full size ----------------
+# ---------------- config 3 (the verify layer) at full size ----------------
 
 def test_config3_moe_verify_layer_full_size():
     """M = 6, d = 4096, E = 512, top-10, I = 1024, q4 G = 128: the whole layer against the oracle. The oracle routes

@@ -1,4 +1,4 @@
-"""BASELINE config 4 at full size on cuda:0 through the C ABI: the MoE layer at prefill width (M = 2048 tokens,
+"""Config 4 at full size on cuda:0 through the C ABI: the MoE layer at prefill width (M = 2048 tokens,
 d = 4096, E = 512, top-10, I = 1024, q4 G = 128, routing skewed by a seeded Zipf(1.1) bias), and the dense linears at
 prefill width (the route the reference's linear_q4_wmma / linear_q8_wmma callers take, kernels/linear_wmma.hpp:22-25).
 

@@ -29,7 +29,7 @@ def rand_qweight(rng, bits, N, K, G):
 
 
 def max_abs_norm_err(got, ref):
-    """max |got - ref| / max |ref|: the north star's 1e-3 tolerance measure."""
+    """max |got - ref| / max |ref|: the measure of the 1e-3 tolerance."""
     got = np.asarray(got, np.float64)
     ref = np.asarray(ref, np.float64)
     return float(np.max(np.abs(got - ref)) / max(np.max(np.abs(ref)), 1e-30))
@@ -76,7 +76,7 @@ def bf16_ulp(r):
 
 
 def assert_close(got, ref, tol=1e-3, what="", roundings=1, max_off_frac=1e-3, max_bias=1e-4):
-    """The north star's bar, plus two checks that catch a systematic error the per-element bound would let through.
+    """The 1e-3 bar, plus two checks that catch a systematic error the per-element bound would let through.
 
     1. Per element: max |got - ref| <= tol * max |ref| (FP32 outputs). BF16 outputs (uint16 bits) may also differ by the
        roundings to BF16 along the way: + roundings * 2^-8 |ref| per element (1: the store; SwiGLU of stored gate and
